@@ -139,9 +139,10 @@ struct Mat
    const int32_t* rowseg;   // NULL when nseg == 1
    const int32_t* colseg;
    const int32_t* perm;     // device row position -> caller's row index
-   const int32_t* rlist;    // rows with two finite sides and at least 3 nonzeros (rowflags bit 1)
+   const int32_t* rlist;    // rows with two finite sides and at least 3 nonzeros (rowflags bit 1),
+                            // first the ngcd of them that hold a gcd-group nonzero (bit 2)
    int32_t nranged;
-   int32_t pad2;
+   int32_t ngcd;
 };
 
 struct Vec
@@ -2574,6 +2575,7 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_history(Mat M, Vec V)
 // yields nothing.
 // ------------------------------------------------------------------------------------------
 #define SAP_RANGED_STEPS (1 << 20)
+#define SAP_GCD_EPS 1e-6   // largest epsilon for which mayBeGcdCoef covers the gcd group
 
 template <bool R>
 __device__ __forceinline__ void rangedCut(const CtxT<R>& C)
@@ -2830,6 +2832,12 @@ __device__ void rangedRow(const Mat& M, const Vec& V, const Params& P, int32_t v
    }
 }
 
+// rows of rlist that the ranged step has to look at under these parameters (mayBeGcdCoef)
+__host__ __device__ __forceinline__ int32_t rangedRows(const Mat& M, const Params& P)
+{
+   return P.epsilon <= SAP_GCD_EPS ? M.ngcd : M.nranged;
+}
+
 // ranged-row step of a round (before the row sweep, on the same start-of-round bounds): the
 // eligible rows marked for this round and not redundant
 template <bool R>
@@ -2842,11 +2850,12 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_ranged(Mat M, Vec V, Params P)
    if( V.dense )
    {
       const bool all = st->firstall && st->rlocal == 1;
-      const size_t n = (size_t)V.nvec * (size_t)M.nranged;
+      const size_t per = (size_t)rangedRows(M, P);
+      const size_t n = (size_t)V.nvec * per;
       for( size_t i = blockIdx.x * (size_t)SAP_BLOCK + threadIdx.x; i < n; i += (size_t)gridDim.x * SAP_BLOCK )
       {
-         const int32_t v = (int32_t)(i / (size_t)M.nranged);
-         const int32_t row = M.rlist[i - (size_t)v * (size_t)M.nranged];
+         const int32_t v = (int32_t)(i / per);
+         const int32_t row = M.rlist[i - (size_t)v * per];
          const size_t rflat = (size_t)v * (size_t)M.nrows + (size_t)row;
          if( (all || V.rowmark[rflat] == round) && !rowRedundant(V, rflat) && (R || !V.vcutoff[unitOfRow(M, v, row)]) )
             rangedRow<R>(M, V, P, v, row);
@@ -2854,6 +2863,7 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_ranged(Mat M, Vec V, Params P)
    }
    else
    {
+      const int flag = rangedRows(M, P) == M.nranged ? 2 : 4;
       for( int b = 0; b < SAP_NBINS; ++b )
       {
          const uint32_t n = st->wlcount[round & 1][b];
@@ -2862,7 +2872,7 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_ranged(Mat M, Vec V, Params P)
          {
             const int2 it = wl[i];
             const size_t rflat = (size_t)it.y * (size_t)M.nrows + (size_t)it.x;
-            if( (M.rowflags[it.x] & 2) && !rowRedundant(V, rflat) && (R || !V.vcutoff[unitOfRow(M, it.y, it.x)]) )
+            if( (M.rowflags[it.x] & flag) && !rowRedundant(V, rflat) && (R || !V.vcutoff[unitOfRow(M, it.y, it.x)]) )
                rangedRow<R>(M, V, P, it.y, it.x);
          }
       }
@@ -3611,6 +3621,7 @@ struct sap_matrix
    int32_t* perm;        // device row position -> caller's row index
    int32_t* rlist;       // device rows eligible for ranged-row propagation
    int32_t nranged;
+   int32_t ngcd;         // the first of them: rows with a nonzero that may join the gcd group
    int32_t binstart[SAP_NBINS + 1];
    int32_t ntiles;
    int64_t* tstart;
@@ -3839,7 +3850,7 @@ static Mat toMat(const sap_matrix* m)
    M.perm = m->perm;
    M.rlist = m->rlist;
    M.nranged = m->nranged;
-   M.pad2 = 0;
+   M.ngcd = m->ngcd;
    return M;
 }
 
@@ -3922,6 +3933,22 @@ static void buildColumns(int64_t nrows, int64_t ncols, int64_t nnz, const int64_
       });
    for( auto& x : th )
       x.join();
+}
+
+// Ranged-row propagation does nothing to a row without an unfixed gcd-group nonzero: an integral
+// column whose coefficient is an integer other than +-1 within epsilon (epsIntegral).  This test
+// of a coefficient is a superset of that one for every epsilon up to SAP_GCD_EPS (the relative
+// term covers the rounding of a + epsilon), so rows in which it holds for no integral column
+// need no ranged step under such an epsilon.  Mixed systems with real coefficients have almost
+// no other rows: a first round's ranged step on 30,000 of them took 336 us (a thread a row,
+// nonzeros read up to three times) and is now not launched; sap_propagate_reasons at a node of
+// that system went from 681 to 272 us.
+// without branches: which nonzeros are integral is random in a large matrix
+static inline int mayBeGcdCoef(double a)
+{
+   const double m = std::min(fabs(a), 0x1p52);   // integers from there on: a fraction of 0
+   const double f = m - (double)(int64_t)m, tol = 2.0 * SAP_GCD_EPS + m * 0x1p-50;
+   return (int)((f <= tol) | (f >= 1.0 - tol)) & (int)(m != 1.0);
 }
 
 static inline int lenBin(int64_t L, int32_t longrow)
@@ -4156,7 +4183,7 @@ static int matrixCreate(sap_context* ctx, int64_t nrows, int64_t ncols, const in
    std::vector<std::array<int64_t, SAP_NBINS>> tcount(16);
    for( auto& c : tcount )
       c.fill(0);
-   parallelFor(nrows, 1 << 16, [&](int64_t i0, int64_t i1, int t) {
+   parallelFor(nrows, 1 << 13, [&](int64_t i0, int64_t i1, int t) {
       std::vector<int32_t> tmp;
       for( int64_t i = i0; i < i1; ++i )
       {
@@ -4262,12 +4289,13 @@ static int matrixCreate(sap_context* ctx, int64_t nrows, int64_t ncols, const in
    std::vector<uint8_t> rowflags((size_t)nrows), rowbin((size_t)nrows);
    std::vector<int64_t> colptr((size_t)ncols + 1);
    HostArray<int32_t> rowidx((size_t)nnz);
-   parallelFor(nrows, 1 << 16, [&](int64_t r0, int64_t r1, int) {
+   parallelFor(nrows, 1 << 13, [&](int64_t r0, int64_t r1, int) {
       for( int64_t r = r0; r < r1; ++r )
       {
          const int64_t i = perm[(size_t)r];
          const int64_t st0 = rowptr[i], L = rowptr[i + 1] - st0, o = prowptr[(size_t)r];
          bool allbin = true;
+         int gcd = 0;
          for( int64_t k = 0; k < L; ++k )
          {
             const int32_t c = colidx[st0 + k];
@@ -4276,12 +4304,13 @@ static int matrixCreate(sap_context* ctx, int64_t nrows, int64_t ncols, const in
             pflag[(size_t)(o + k)] = colflags[(size_t)c];
             if( !(colflags[(size_t)c] & 2) )
                allbin = false;
+            gcd |= (colflags[(size_t)c] & 1) & mayBeGcdCoef(vals[st0 + k]);
          }
          sides[(size_t)r] = make_double2(lhs[i], rhs[i]);
          // bit 1: eligible for ranged-row propagation (two sides of magnitude below SCIP's
          // default infinity, at least 3 nonzeros)
          const bool ranged = L >= 3 && fabs(lhs[i]) < 1e20 && fabs(rhs[i]) < 1e20;
-         rowflags[(size_t)r] = (uint8_t)((allbin ? 1 : 0) | (ranged ? 2 : 0));
+         rowflags[(size_t)r] = (uint8_t)((allbin ? 1 : 0) | (ranged ? 2 : 0) | (ranged && gcd ? 4 : 0));
          rowbin[(size_t)r] = obin[(size_t)i];
       }
    });
@@ -4347,10 +4376,12 @@ static int matrixCreate(sap_context* ctx, int64_t nrows, int64_t ncols, const in
    m->nrows = nrows;
    m->ncols = ncols;
    m->nnz = nnz;
-   std::vector<int32_t> rlist;
+   std::vector<int32_t> rlist, others;
    for( int64_t r = 0; r < nrows; ++r )
       if( rowflags[(size_t)r] & 2 )
-         rlist.push_back((int32_t)r);
+         ((rowflags[(size_t)r] & 4) ? rlist : others).push_back((int32_t)r);
+   m->ngcd = (int32_t)rlist.size();
+   rlist.insert(rlist.end(), others.begin(), others.end());
    m->nranged = (int32_t)rlist.size();
    // ranged-row propagation submits forced candidates, so matrices with eligible rows keep them
    m->hasforced = hasforced || m->nranged > 0;
@@ -5012,10 +5043,11 @@ static void enqueueRound(sap_bounds* b, const Mat& M, const Params& P, const Lay
    const unsigned colgrid = gridFor((size_t)b->V.nvec * (size_t)m->ncols, 4096);
    if( !begun )
       k_round_begin<<<1, SAP_STAT_SLOTS, 0, s>>>(b->V, P.maxrounds);
-   if( (P.flags & SAP_FLAG_RANGEDROWS) && m->nranged > 0 && b->V.reasons )
-      k_ranged<true><<<gridFor((size_t)b->V.nvec * (size_t)m->nranged, 4096), SAP_BLOCK, 0, s>>>(M, b->V, P);
-   else if( (P.flags & SAP_FLAG_RANGEDROWS) && m->nranged > 0 )
-      k_ranged<false><<<gridFor((size_t)b->V.nvec * (size_t)m->nranged, 4096), SAP_BLOCK, 0, s>>>(M, b->V, P);
+   const int32_t nranged = (P.flags & SAP_FLAG_RANGEDROWS) ? rangedRows(M, P) : 0;
+   if( nranged > 0 && b->V.reasons )
+      k_ranged<true><<<gridFor((size_t)b->V.nvec * (size_t)nranged, 4096), SAP_BLOCK, 0, s>>>(M, b->V, P);
+   else if( nranged > 0 )
+      k_ranged<false><<<gridFor((size_t)b->V.nvec * (size_t)nranged, 4096), SAP_BLOCK, 0, s>>>(M, b->V, P);
    if( e0 != NULL )
       (void)hipEventRecord(e0, s);
    if( nsweep > 0 && b->V.reasons )

@@ -54,6 +54,38 @@ def test_large_system(gpu_ctx, seed):
     check(gpu_ctx, inst, f"large{seed}")
 
 
+@pytest.mark.parametrize("eps", [1e-9, 1e-6, 1e-5, 1e-3])
+def test_coefficients_near_integers(gpu_ctx, eps):
+    # which rows hold a gcd-group coefficient depends on epsilon: coefficients an integer off by
+    # less than, about and more than it, rows of real coefficients and magnitudes where a unit in
+    # the last place exceeds it, among rows that have nothing to do with the gcd step
+    rng = np.random.default_rng(1320)
+    cut = differs = 0
+    for i in range(40):
+        inst = ranged_system(np.random.default_rng(1330 + i), 5, 12, slack=False)
+        off = rng.choice([4e-10, 9e-7, -9e-7, 2.5e-6, 5e-4, 0.3, 1e12], size=inst.nnz)
+        inst.vals[:] += np.where(rng.random(inst.nnz) < 0.15, off, 0.0)
+        say(f"[case] ranged near-integer coefficients eps={eps} inst={i}")
+        om = orc.OMatrix.from_instance(inst)
+        ol, ou, orr = orc.propagate_jacobi(om, inst.lb, inst.ub, orc.params(rangedrows=1, epsilon=eps))
+        _, _, plain = orc.propagate_jacobi(om, inst.lb, inst.ub, orc.params(rangedrows=0, epsilon=eps))
+        cut += orr["cutoff"]
+        differs += orr["cutoff"] != plain["cutoff"] or orr["nchgbds"] != plain["nchgbds"]
+        mat = sa.Matrix(gpu_ctx, inst)
+        for mode in (sa.SAP_MODE_DENSE, sa.SAP_MODE_SPARSE):
+            b = sa.Bounds(mat, 1, mode)
+            b.upload(inst.lb, inst.ub)
+            st = b.propagate(sa.default_params(flags=RANGED, epsilon=eps))
+            assert (st["result"] == sa.SAP_CUTOFF) == bool(orr["cutoff"]), (i, mode)
+            if not orr["cutoff"]:
+                gl, gu = b.download(0)
+                assert np.array_equal(gl, ol) and np.array_equal(gu, ou), (i, mode)
+                assert st["nchgbds"] == orr["nchgbds"]
+            b.close()
+        mat.close()
+    assert 0 < cut < 40 and differs > 5   # the ranged step matters in these systems
+
+
 @pytest.mark.parametrize("seed", range(2))
 def test_mixed(gpu_ctx, seed):
     check(gpu_ctx, sa.gen_mixed(20000, 20000, seed=70 + seed, planted=True), f"mixed{seed}")
