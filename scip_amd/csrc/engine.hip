@@ -52,12 +52,20 @@ using namespace sap;
 #define SAP_MAXLEVELS 40
 #define SAP_ROUND_CAP 10000000
 #define SAP_STAT_SLOTS 256
+#define SAP_CHG_SAMPLE 16   // statistics slots that the marking reads (one cache line)
 
 // row-length bins: 0 empty rows; 1..5 at most 4,8,16,32,64 nonzeros (tiles in dense mode,
 // groups of 4,8,16,32,64 lanes in sparse mode); 6 at most 128 nonzeros (tiles of width 2 in
 // dense mode, else a wavefront per row); 7 wavefront per row; 8 workgroup per row (rows longer
 // than the tuning's longrow, from any of bins 6..8)
 static const int32_t kBinMaxLen[SAP_NBINS - 2] = { 0, 4, 8, 16, 32, 64, 128 };
+
+// a list length that many workgroups add to, on a cache line of its own: additions to one line
+// serialise at 15-20 ns each, also when they go to different words of it
+struct alignas(128) Counter
+{
+   uint32_t n;
+};
 
 struct Status
 {
@@ -68,9 +76,12 @@ struct Status
    int32_t firstall;    // dense mode: the first round of the call sweeps every row
    int32_t anymark[2];  // dense mode: some row is marked for the round of this parity
    int32_t rgenm1;      // generation of the locally-redundant row flags, minus one (redGen)
-   uint32_t wlcount[2][SAP_NBINS];   // sparse mode worklist lengths
-   uint32_t touched;                 // sparse mode touched-column count
-   uint32_t pad2;
+   // dense mode: the rows marked for the round of this parity are all in its worklists, unless
+   // some did not fit
+   int32_t listed[2];
+   int32_t listovf[2];
+   Counter wlcount[2][SAP_NBINS];    // worklist lengths (what did not fit is counted too)
+   Counter touched;                  // touched-column count (likewise)
    unsigned long long rows_swept;
    unsigned long long nnz_swept;
    unsigned long long nchg;
@@ -79,6 +90,7 @@ struct Status
    unsigned long long slot_nnz[SAP_STAT_SLOTS];
    unsigned long long slot_rows[SAP_STAT_SLOTS];
    unsigned long long slot_chg[SAP_STAT_SLOTS];
+   unsigned long long chgbase;       // the sum of the first SAP_CHG_SAMPLE at the start of the round
    // sweep launch duration from the constant-rate wall clock: earliest workgroup start and
    // latest workgroup end per slot, folded at the end of the round
    unsigned long long tslot0[SAP_STAT_SLOTS];
@@ -171,8 +183,15 @@ struct Vec
    int32_t* ovln;           // per vector
    int32_t logchg;          // record changed columns
    int32_t nseg;            // segments of the matrix (units per vector)
-   int2* wl[2][SAP_NBINS];  // sparse mode: (row, vector) worklists, double-buffered by round parity
-   int2* touched;           // sparse mode: (column, vector)
+   // worklists: (row, vector) per length bin, double-buffered by round parity, and (column,
+   // vector) with a candidate.  Sparse mode keeps them in every round and has room for all;
+   // dense mode uses them in rounds that few changed columns lead to (markRound)
+   int2* wl[2][SAP_NBINS];
+   int2* touched;
+   uint32_t listcap;        // entries of each worklist
+   uint32_t touchcap;
+   uint32_t listper;        // dense mode, per vector: changed columns up to which rows are listed
+   uint32_t pad6;
    Status* st;
    // reason recording (one vector, one instance): every candidate that reaches or ties the
    // running best of its column goes to the round's candidate log; the column step notes
@@ -436,7 +455,7 @@ __device__ __forceinline__ uint64_t laneMaskLt()
    return lane == 0 ? 0ULL : (~0ULL >> (64 - lane));
 }
 
-__device__ __forceinline__ void waveAppendTouched(Status* st, int2* list, bool pred, int2 item)
+__device__ __forceinline__ void waveAppendTouched(const Vec& V, bool pred, int2 item)
 {
    const uint64_t m = __ballot(pred);
    if( m == 0 )
@@ -445,10 +464,11 @@ __device__ __forceinline__ void waveAppendTouched(Status* st, int2* list, bool p
    const int lane = (int)threadIdx.x & (SAP_WAVE - 1);
    uint32_t base = 0;
    if( lane == leader )
-      base = atomicAdd(&st->touched, (uint32_t)__popcll(m));
+      base = atomicAdd(&V.st->touched.n, (uint32_t)__popcll(m));
    base = __shfl(base, leader, SAP_WAVE);
-   if( pred )
-      list[base + __popcll(m & laneMaskLt())] = item;
+   const uint32_t at = base + (uint32_t)__popcll(m & laneMaskLt());
+   if( pred && at < V.touchcap )
+      V.touched[at] = item;
 }
 
 __device__ __forceinline__ void waveAppendRow(Status* st, int2* const* wl, int npar, bool pred, int bin, int2 item)
@@ -463,7 +483,7 @@ __device__ __forceinline__ void waveAppendRow(Status* st, int2* const* wl, int n
       const uint64_t grp = __ballot(mine);
       uint32_t base = 0;
       if( lane == leader )
-         base = atomicAdd(&st->wlcount[npar][lbin], (uint32_t)__popcll(grp));
+         base = atomicAdd(&st->wlcount[npar][lbin].n, (uint32_t)__popcll(grp));
       base = __shfl(base, leader, SAP_WAVE);
       if( mine )
       {
@@ -474,29 +494,56 @@ __device__ __forceinline__ void waveAppendRow(Status* st, int2* const* wl, int n
    }
 }
 
-// one pass of (row, vector) worklist appends by a whole workgroup of SAP_BLOCK threads: the
-// fresh rows are counted per length bin in LDS (scnt, sbase: SAP_NBINS entries each) and
-// appended with one global atomic per bin.  Every thread of the workgroup calls it (barriers
-// inside).  scnt[t] is cleared by thread t, which also was its only reader in the previous
-// pass; sbase is rewritten only after the second barrier, which every reader of the previous
-// pass has passed.
-__device__ __forceinline__ void blockAppendRows(Status* st, int2* const* wl, int npar, bool fresh, int bin,
-   int2 item, uint32_t* scnt, uint32_t* sbase)
+// exclusive sum of one number per thread of a workgroup of SAP_BLOCK threads, and the total
+// (wsum: one LDS entry per wavefront; barriers inside)
+__device__ __forceinline__ int64_t blockScan(int64_t x, int64_t* wsum, int64_t& total)
 {
-   const int t = (int)threadIdx.x;
-   if( t < SAP_NBINS )
-      scnt[t] = 0;
+   const int lane = (int)threadIdx.x & (SAP_WAVE - 1);
+   const int wave = (int)threadIdx.x / SAP_WAVE;
+   int64_t inc = x;
+#pragma unroll
+   for( int d = 1; d < SAP_WAVE; d <<= 1 )
+   {
+      const int64_t add = __shfl_up((long long)inc, d, SAP_WAVE);
+      if( lane >= d )
+         inc += add;
+   }
+   __syncthreads();   // the previous use of wsum has been read
+   if( lane == SAP_WAVE - 1 )
+      wsum[wave] = inc;
    __syncthreads();
-   uint32_t pos = 0;
-   if( fresh )
-      pos = atomicAdd(&scnt[bin], 1u);
-   __syncthreads();
-   if( t < SAP_NBINS && scnt[t] > 0 )
-      sbase[t] = atomicAdd(&st->wlcount[npar][t], scnt[t]);
-   __syncthreads();
-   if( fresh )
-      wl[bin][sbase[bin] + pos] = item;
+   int64_t before = 0;
+   total = 0;
+#pragma unroll
+   for( int w = 0; w < SAP_BLOCK / SAP_WAVE; ++w )
+   {
+      before += w < wave ? wsum[w] : 0;
+      total += wsum[w];
+   }
+   return before + inc - x;
 }
+
+// LDS of blockMark
+struct MarkShared
+{
+   int64_t off[SAP_BLOCK + 1];   // off[k]: rows of the workgroup's columns before thread k's
+   int64_t beg[SAP_BLOCK];       // colptr of thread k's column
+   int32_t vec[SAP_BLOCK];       // its vector
+   int64_t wsum[SAP_BLOCK / SAP_WAVE];
+   uint32_t cnt[SAP_NBINS];      // fresh rows of one pass per length bin
+   uint32_t base[SAP_NBINS];     // their first worklist position
+};
+
+// rows marked for round `first` and appended to its worklists by a whole workgroup: thread t's
+// column has the rows rowidx[beg .. beg + len) in vector v (len 0: no column).  The rows are
+// numbered across the workgroup, so that every thread takes the next one whatever the column
+// lengths; SAP_MARK_ROWS per thread and pass are tagged first, then the fresh ones counted per
+// length bin in LDS and appended with one global atomic per bin.  What bounds it is the chain
+// of a pass (row index, tag, bin, LDS count, append), so a pass is long.  skipred: rows that
+// are locally redundant are not marked.
+#define SAP_MARK_ROWS 4
+__device__ __forceinline__ void blockMark(const Mat& M, const Vec& V, MarkShared& S, int64_t beg, int64_t len,
+   int32_t v, int32_t first, bool skipred, bool& any);
 
 // ------------------------------------------------------------------------------------------
 // candidates
@@ -529,6 +576,115 @@ __device__ __forceinline__ bool rowRedundant(const Vec& V, size_t rflat)
    return V.redundant[rflat] == redGen(V);
 }
 
+__device__ __forceinline__ void blockMark(const Mat& M, const Vec& V, MarkShared& S, int64_t beg, int64_t len,
+   int32_t v, int32_t first, bool skipred, bool& any)
+{
+   Status* st = V.st;
+   const int t = (int)threadIdx.x;
+   const int par = first & 1;
+   const uint8_t gen = redGen(V);
+   int64_t total;
+   const int64_t mine = blockScan(len, S.wsum, total);
+   S.off[t] = mine;
+   S.beg[t] = beg;
+   S.vec[t] = v;
+   if( t == 0 )
+      S.off[SAP_BLOCK] = total;
+   __syncthreads();
+   // passes are workgroup-uniform: total is the same in every thread
+   for( int64_t f0 = 0; f0 < total; f0 += SAP_MARK_ROWS * SAP_BLOCK )
+   {
+      int2 item[SAP_MARK_ROWS];
+      int bin[SAP_MARK_ROWS];
+      uint32_t pos[SAP_MARK_ROWS];
+      if( t < SAP_NBINS )
+         S.cnt[t] = 0;   // thread t was its only reader in the previous pass
+#pragma unroll
+      for( int k = 0; k < SAP_MARK_ROWS; ++k )
+      {
+         const int64_t f = f0 + k * SAP_BLOCK + t;
+         bin[k] = -1;
+         item[k] = make_int2(0, 0);
+         if( f < total )
+         {
+            // the column of row f: the largest k with off[k] <= f, which has off[k + 1] > f
+            int lo = 0, hi = SAP_BLOCK - 1;
+            while( lo < hi )
+            {
+               const int mid = (lo + hi + 1) >> 1;
+               if( S.off[mid] <= f )
+                  lo = mid;
+               else
+                  hi = mid - 1;
+            }
+            const int32_t rv = S.vec[lo];
+            const int32_t row = M.rowidx[S.beg[lo] + (f - S.off[lo])];
+            const size_t rflat = (size_t)rv * (size_t)M.nrows + (size_t)row;
+            if( !skipred || V.redundant[rflat] != gen )
+            {
+               if( V.vpend[rv] != first )
+                  V.vpend[rv] = first;   // every writer of this round stores the same value
+               any = true;
+               if( atomicMax(&V.rowmark[rflat], first) < first )
+                  bin[k] = M.rowbin[row];
+               item[k] = make_int2(row, rv);
+            }
+         }
+      }
+      __syncthreads();
+#pragma unroll
+      for( int k = 0; k < SAP_MARK_ROWS; ++k )
+         pos[k] = bin[k] >= 0 ? atomicAdd(&S.cnt[bin[k]], 1u) : 0;
+      __syncthreads();
+      if( t < SAP_NBINS && S.cnt[t] > 0 )
+      {
+         S.base[t] = atomicAdd(&st->wlcount[par][t].n, S.cnt[t]);
+         if( S.base[t] + S.cnt[t] > V.listcap )
+            st->listovf[par] = 1;   // dense mode: the round scans the row tags instead
+      }
+      __syncthreads();
+#pragma unroll
+      for( int k = 0; k < SAP_MARK_ROWS; ++k )
+         if( bin[k] >= 0 && S.base[bin[k]] + pos[k] < V.listcap )
+            V.wl[par][bin[k]][S.base[bin[k]] + pos[k]] = item[k];
+   }
+   __syncthreads();   // S is rewritten by the next columns
+}
+
+// the round's control fields, loaded together at the start of a kernel: one wait instead of one
+// per test (each is 0.5-1 us at the start of every workgroup)
+struct RoundView
+{
+   int32_t round;
+   int32_t rlocal;
+   int32_t done;
+   int32_t cutoff;
+   int32_t firstall;
+   // the round is swept from worklists: always in sparse mode; in dense mode when the marking
+   // that led to it listed every row.  Nothing in the round itself changes the answer.
+   bool listed;
+   // ... and (after the sweep) its columns with a candidate are all in the touched list
+   bool columns;
+   uint32_t touched;
+};
+
+__device__ __forceinline__ RoundView roundView(const Vec& V)
+{
+   const Status* st = V.st;
+   RoundView r;
+   r.round = st->round;
+   r.rlocal = st->rlocal;
+   r.done = st->done;
+   r.cutoff = st->cutoff;
+   r.firstall = st->firstall;
+   const int32_t l0 = st->listed[0], l1 = st->listed[1], o0 = st->listovf[0], o1 = st->listovf[1];
+   r.touched = st->touched.n;
+   const bool odd = (r.round & 1) != 0;
+   r.listed = !V.dense || ((odd ? l1 : l0) && !(odd ? o1 : o0));
+   r.columns = r.listed && r.touched <= V.touchcap;
+   return r;
+}
+
 __device__ __forceinline__ int32_t unitOfRow(const Mat& M, int32_t v, int32_t row)
 {
    return M.rowseg == NULL ? v : v * M.nseg + M.rowseg[row];
@@ -551,7 +707,7 @@ __device__ __forceinline__ void touch(const CtxT<R>& C, size_t flat, int32_t j)
    else
    {
       const bool first = atomicMax(&C.V->coltag[flat], C.round) < C.round;
-      waveAppendTouched(C.V->st, C.V->touched, first, make_int2(j, C.v));
+      waveAppendTouched(*C.V, first, make_int2(j, C.v));
    }
 }
 
@@ -1984,30 +2140,81 @@ __device__ __forceinline__ void blockStats(unsigned long long a, unsigned long l
    }
 }
 
-template <bool R>
+// a listed round's workgroups are shared out over the length bins by the passes that the bins'
+// lists need (rows per workgroup and pass: 2^shift), so that short lists spread over the chip
+// and a long one gets what is left.  false: nothing for this workgroup.
+__device__ __forceinline__ bool listShare(const Mat& M, const Status& st, int par, int& kind, int& lblock, int& nblocks)
+{
+   constexpr int kShift[SAP_NBINS] = { 6, 6, 5, 4, 3, 2, 2, 2, 0 };
+   const uint32_t grid = gridDim.x;
+   uint32_t need[SAP_NBINS], total = 0;
+#pragma unroll
+   for( int b = 0; b < SAP_NBINS; ++b )
+   {
+      const int sh = (b >= 1 && b <= M.rowbins) ? 8 : kShift[b];
+      need[b] = (uint32_t)(((uint64_t)st.wlcount[par][b].n + (1u << sh) - 1) >> sh);
+      total += need[b];
+   }
+   uint32_t start = 0;
+   bool found = false;
+#pragma unroll
+   for( int b = 0; b < SAP_NBINS; ++b )
+   {
+      uint32_t n = need[b];
+      if( total > grid && n > 0 )
+      {
+         n = (uint32_t)((uint64_t)n * (grid - SAP_NBINS) / total);   // grid >= SAP_LISTGRID
+         n = n > 0 ? n : 1;
+      }
+      if( !found && blockIdx.x < start + n )
+      {
+         kind = 1 + b;
+         lblock = (int)(blockIdx.x - start);
+         nblocks = (int)n;
+         found = true;
+      }
+      start += n;
+   }
+   return found;
+}
+
+// D: a dense bound set (its rounds are scanned or listed); a sparse one's rounds are all listed,
+// and its kernel carries none of the tile code
+template <bool R, bool D>
 __global__ __launch_bounds__(SAP_BLOCK, 4) void k_sweep(Mat M, Vec V, Params P, Layout L)
 {
    Status* st = V.st;
-   if( st->done )
+   const RoundView rv = roundView(V);
+   if( rv.done )
       return;
    const unsigned long long tstart = (unsigned long long)wall_clock64();
    if( threadIdx.x == 0 )
       s_nrecomp = 0;
    __syncthreads();
-   const int blk = (int)blockIdx.x;
-   int kind = 0;
-   while( kind < SAP_NKINDS - 1 && blk >= L.blockstart[kind + 1] )
-      ++kind;
-   const int lblock = blk - L.blockstart[kind];
-   const int nblocks = L.blockstart[kind + 1] - L.blockstart[kind];
-   const int b = kind - 1;   // row-length bin (kind 0: tiles)
    Items I;
-   I.round = st->round;
-   I.rlocal = st->rlocal;
-   I.firstall = (V.dense && st->firstall && I.rlocal == 1) ? 1 : 0;
+   I.round = rv.round;
+   // W: this round's form (W.dense: row and column tags are scanned; else lists are kept)
+   Vec W = V;
+   W.dense = (D && !rv.listed) ? 1 : 0;
+   int kind = 0, lblock, nblocks;
+   if( D && W.dense )
+   {
+      const int blk = (int)blockIdx.x;
+      while( kind < SAP_NKINDS - 1 && blk >= L.blockstart[kind + 1] )
+         ++kind;
+      lblock = blk - L.blockstart[kind];
+      nblocks = L.blockstart[kind + 1] - L.blockstart[kind];
+      if( lblock >= nblocks )
+         return;   // a workgroup that only listed rounds use
+   }
+   else if( !listShare(M, *st, I.round & 1, kind, lblock, nblocks) )
+      return;
+   const int b = kind - 1;   // row-length bin (kind 0: tiles)
+   I.rlocal = rv.rlocal;
+   I.firstall = (W.dense && rv.firstall && I.rlocal == 1) ? 1 : 0;
    I.binbase = b >= 0 ? M.binstart[b] : 0;
    I.binlen = b >= 0 ? M.binstart[b + 1] - M.binstart[b] : 0;
-   if( V.dense )
+   if( W.dense )
    {
       I.list = NULL;
       I.n = (uint32_t)V.nvec * (uint32_t)I.binlen;
@@ -2015,7 +2222,7 @@ __global__ __launch_bounds__(SAP_BLOCK, 4) void k_sweep(Mat M, Vec V, Params P, 
    else
    {
       I.list = b >= 0 ? V.wl[I.round & 1][b] : NULL;
-      I.n = b >= 0 ? st->wlcount[I.round & 1][b] : 0;
+      I.n = b >= 0 ? st->wlcount[I.round & 1][b].n : 0;
    }
    unsigned long long nnzacc = 0, rowsacc = 0;
    constexpr int NW = SAP_BLOCK / SAP_WAVE;
@@ -2048,12 +2255,14 @@ __global__ __launch_bounds__(SAP_BLOCK, 4) void k_sweep(Mat M, Vec V, Params P, 
    switch( kind )
    {
    case 0:
+      if constexpr( !D )
+         break;   // only scanned rounds have tiles
       if( M.twidth == 2 )
-         sweepTilesW<R, 2>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepTilesW<R, 2>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       else if( M.twidth == 4 )
-         sweepTilesW<R, 4>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepTilesW<R, 4>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       else
-         sweepTiles<R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepTiles<R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       // empty rows (first round only; they are never marked again): activity 0 against the
       // sides, propagateCons's infeasibility test (cons_linear.c:7721-7742)
       if( I.firstall && lblock == 0 )
@@ -2076,34 +2285,34 @@ __global__ __launch_bounds__(SAP_BLOCK, 4) void k_sweep(Mat M, Vec V, Params P, 
             rowsacc += (unsigned long long)V.nvec * (unsigned long long)nempty;
       }
       break;
-   case 1: sweepGroups<4, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
+   case 1: sweepGroups<4, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
    case 2:
       if( M.rowbins >= 1 )
-         sweepRows<4, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepRows<4, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       else
-         sweepGroups<4, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepGroups<4, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       break;
    case 3:
       if( M.rowbins >= 2 )
-         sweepRows<8, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepRows<8, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       else
-         sweepGroups<8, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepGroups<8, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       break;
    case 4:
       if( M.rowbins >= 3 )
-         sweepRows<16, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepRows<16, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       else
-         sweepGroups<16, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
+         sweepGroups<16, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q);
       break;
-   case 5: sweepGroups<32, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
-   case 6: sweepGroups<64, R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
+   case 5: sweepGroups<32, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
+   case 6: sweepGroups<64, R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
    case 7:
-   case 8: sweepWaves<R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
-   default: sweepBlocks<R>(M, V, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
+   case 8: sweepWaves<R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
+   default: sweepBlocks<R>(M, W, P, I, lblock, nblocks, nnzacc, rowsacc, Q); break;
    }
    // remaining queued candidates of this wavefront
    if( Q.count > 0 )
-      drainQueue<R>(M, V, P, Q, Q.count, I.round);
+      drainQueue<R>(M, W, P, Q, Q.count, I.round);
    blockStats(nnzacc, rowsacc, st->slot_nnz, st->slot_rows);   // ends with a barrier
    if( threadIdx.x == 0 )
    {
@@ -2280,10 +2489,12 @@ __device__ __forceinline__ int columnStep(const Mat& M, const Vec& V, const Para
 // of one workgroup)
 __device__ __forceinline__ void foldStamps(Status* st)
 {
-   __shared__ unsigned long long tmin[SAP_STAT_SLOTS], tmax[SAP_STAT_SLOTS];
+   __shared__ unsigned long long tmin[SAP_STAT_SLOTS], tmax[SAP_STAT_SLOTS], chg[SAP_CHG_SAMPLE];
    const int t = (int)threadIdx.x;
    tmin[t] = st->tslot0[t];
    tmax[t] = st->tslot1[t];
+   if( t < SAP_CHG_SAMPLE )
+      chg[t] = st->slot_chg[t];
    st->tslot0[t] = ~0ULL;
    st->tslot1[t] = 0;
    __syncthreads();
@@ -2295,6 +2506,13 @@ __device__ __forceinline__ void foldStamps(Status* st)
          tmax[t] = tmax[t] > tmax[t + w] ? tmax[t] : tmax[t + w];
       }
       __syncthreads();
+   }
+   if( t == 0 )
+   {
+      unsigned long long sum = 0;
+      for( int q = 0; q < SAP_CHG_SAMPLE; ++q )
+         sum += chg[q];
+      st->chgbase = sum;   // what the coming round's marking subtracts (markRound)
    }
    if( t == 0 && tmin[0] != ~0ULL && tmax[0] >= tmin[0] )
    {
@@ -2317,61 +2535,47 @@ __host__ __device__ __forceinline__ bool stopsNext(const Status& st, bool dense,
    {
       uint32_t in = 0;
       for( int b = 0; b < SAP_NBINS; ++b )
-         in += st.wlcount[r & 1][b];
+         in += st.wlcount[r & 1][b].n;
       more = in != 0;
    }
    return !more || st.cutoff || (!st.cont && maxrounds >= 0 && st.rlocal >= maxrounds);
 }
 
-// mark the rows of a changed column for the next round (eventExecLinear marks them)
-__device__ __forceinline__ void markColumn(const Mat& M, const Vec& V, int32_t j, int32_t v, int32_t next, int npar,
+// mark the rows of a changed column for the next round (eventExecLinear marks them) by their
+// tags alone
+__device__ __forceinline__ void markColumn(const Mat& M, const Vec& V, int32_t j, int32_t v, int32_t next,
    bool& anymarked)
 {
-   Status* st = V.st;
-   if( V.dense )
-   {
-      // Round tags are stored without being read first, also on locally redundant rows, which
-      // the dense sweep skips.  Whether the vector has a non-redundant row marked for the
-      // round (its pending round, the round's "any row marked") reads the redundant flags
-      // only until such a row is known.
-      bool known = V.vpend[v] == next;
-      for( int64_t q = M.colptr[j]; q < M.colptr[j + 1]; ++q )
-      {
-         const size_t rflat = (size_t)v * (size_t)M.nrows + (size_t)M.rowidx[q];
-         V.rowmark[rflat] = next;
-         if( !known && !rowRedundant(V, rflat) )
-            known = true;
-      }
-      if( known )
-      {
-         if( V.vpend[v] != next )
-            V.vpend[v] = next;   // every writer of this round stores the same value
-         anymarked = true;
-      }
-      return;
-   }
+   // Round tags are stored without being read first, also on locally redundant rows, which
+   // the dense sweep skips.  Whether the vector has a non-redundant row marked for the
+   // round (its pending round, the round's "any row marked") reads the redundant flags
+   // only until such a row is known.
+   bool known = V.vpend[v] == next;
    for( int64_t q = M.colptr[j]; q < M.colptr[j + 1]; ++q )
    {
-      const int32_t row = M.rowidx[q];
-      const size_t rflat = (size_t)v * (size_t)M.nrows + (size_t)row;
-      if( rowRedundant(V, rflat) )
-         continue;
+      const size_t rflat = (size_t)v * (size_t)M.nrows + (size_t)M.rowidx[q];
+      V.rowmark[rflat] = next;
+      if( !known && !rowRedundant(V, rflat) )
+         known = true;
+   }
+   if( known )
+   {
       if( V.vpend[v] != next )
          V.vpend[v] = next;   // every writer of this round stores the same value
-      const bool first = atomicMax(&V.rowmark[rflat], next) < next;
-      waveAppendRow(st, V.wl[npar], npar, first, M.rowbin[row], make_int2(row, v));
+      anymarked = true;
    }
 }
 
 __global__ __launch_bounds__(SAP_BLOCK) void k_columns(Mat M, Vec V, Params P)
 {
    Status* st = V.st;
-   if( st->done )
+   const RoundView rv = roundView(V);
+   if( rv.done )
       return;
-   const int32_t round = st->round;
+   const int32_t round = rv.round;
    const int32_t next = round + 1;
    unsigned long long nchg = 0;
-   if( V.dense )
+   if( !rv.columns )
    {
       const size_t n = (size_t)V.nvec * (size_t)M.ncols;
       for( size_t flat = blockIdx.x * (size_t)SAP_BLOCK + threadIdx.x; flat < n; flat += (size_t)gridDim.x * SAP_BLOCK )
@@ -2385,7 +2589,7 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_columns(Mat M, Vec V, Params P)
    }
    else
    {
-      const uint32_t n = st->touched;
+      const uint32_t n = rv.touched;
       for( uint32_t idx = blockIdx.x * SAP_BLOCK + threadIdx.x; idx < n; idx += gridDim.x * SAP_BLOCK )
       {
          const int2 t = V.touched[idx];
@@ -2397,116 +2601,146 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_columns(Mat M, Vec V, Params P)
 
 // second half of the column step: rows of the columns changed in this round are marked for the
 // next one, unless their unit was cut off in the round (acceptance and marking are separate
-// launches so that a round ending in infeasibility marks nothing)
+// launches so that a round ending in infeasibility marks nothing).
+//
+// Sparse mode lists the marked rows.  Dense mode tags them, and lists them too when the round
+// changed few columns (at most listper per vector: about 1/64 of the rows marked): a
+// listed round sweeps its rows, steps its touched columns and marks from those, where a
+// scanned one visits every tile, column and tag.  More marked rows than that are swept faster
+// in full tiles, and listing them costs more than it gives (every row's tag is then read
+// back).
+#define SAP_MARK_BLOCKS 512   // workgroups that list rows (an atomic per workgroup and length bin)
+#define SAP_MARK_FLATS (4 * SAP_BLOCK)
+
 __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
 {
    Status* st = V.st;
-   const int32_t round = st->round;
+   const RoundView rv = roundView(V);
+   // changed bounds of this round, estimated from the column step's first statistics slots (its
+   // workgroup w counts in slot w modulo SAP_STAT_SLOTS, and its grid is this one): reading
+   // all of them, with the barriers that takes, cost every scanned round 5-7 us
+   unsigned long long changed = 0;
+#pragma unroll
+   for( int q = 0; q < SAP_CHG_SAMPLE; ++q )
+      changed += st->slot_chg[q];
+   changed -= st->chgbase;
+   if( rv.done || (V.single && rv.cutoff) )
+      return;
+   __shared__ MarkShared S;
+   __shared__ uint32_t found[SAP_BLOCK + SAP_MARK_FLATS];
+   __shared__ uint32_t nfound;
+   const int t = (int)threadIdx.x;
+   const int32_t round = rv.round;
    const int32_t next = round + 1;
-   const int npar = next & 1;
    bool anymarked = false;
-   if( V.dense )
+   bool list = true;
+   if( rv.columns )
    {
-      const size_t n = (size_t)V.nvec * (size_t)M.ncols;
-      for( size_t flat = blockIdx.x * (size_t)SAP_BLOCK + threadIdx.x; flat < n; flat += (size_t)gridDim.x * SAP_BLOCK )
+      const uint32_t n = rv.touched;
+      list = !V.dense || (uint64_t)n <= (uint64_t)V.listper * (uint64_t)V.nvec;
+      // the loop is workgroup-uniform: st->touched is not written in this launch
+      for( uint32_t c0 = blockIdx.x * SAP_BLOCK; c0 < n; c0 += gridDim.x * SAP_BLOCK )
       {
-         if( V.chgtag[flat] != round )
+         int64_t len = 0, beg = 0;
+         int32_t v = 0, j = 0;
+         bool chg = false;
+         if( c0 + (uint32_t)t < n )
+         {
+            const int2 e = V.touched[c0 + (uint32_t)t];
+            j = e.x;
+            v = e.y;
+            chg = V.chgtag[(size_t)v * (size_t)M.ncols + (size_t)j] == round && V.vcutoff[unitOfCol(M, v, j)] == 0;
+         }
+         if( !list )
+         {
+            if( chg )
+               markColumn(M, V, j, v, next, anymarked);
             continue;
-         const int32_t v = (int32_t)(flat / (size_t)M.ncols);
-         const int32_t j = (int32_t)(flat - (size_t)v * (size_t)M.ncols);
-         if( V.vcutoff[unitOfCol(M, v, j)] == 0 )
-            markColumn(M, V, j, v, next, npar, anymarked);
+         }
+         if( chg )
+         {
+            beg = M.colptr[j];
+            len = M.colptr[j + 1] - beg;
+         }
+         blockMark(M, V, S, beg, len, v, next, true, anymarked);
       }
    }
    else
    {
-      // The touched entries are taken SAP_BLOCK at a time.  The rows of the changed columns
-      // among them are numbered across the workgroup (a scan of the column lengths in LDS),
-      // so a wavefront appends up to 64 rows to the worklists at once instead of one append
-      // per row of its longest column.  st->touched is not written in this launch, so the
-      // loop around the barriers is workgroup-uniform.
-      __shared__ int64_t soff[SAP_BLOCK + 1];   // soff[k]: rows of the chunk's columns before entry k
-      __shared__ int64_t sbeg[SAP_BLOCK];       // colptr of entry k's column
-      __shared__ int32_t svec[SAP_BLOCK];       // entry k's vector
-      __shared__ uint32_t scnt[SAP_NBINS];
-      __shared__ uint32_t sbase[SAP_NBINS];
-      const int t = (int)threadIdx.x;
-      const uint32_t n = st->touched;
-      for( uint32_t c0 = blockIdx.x * SAP_BLOCK; c0 < n; c0 += gridDim.x * SAP_BLOCK )
+      const unsigned used = gridDim.x < SAP_STAT_SLOTS ? gridDim.x : SAP_STAT_SLOTS;
+      const unsigned scale = used > SAP_CHG_SAMPLE ? used / SAP_CHG_SAMPLE : 1;
+      list = changed * scale <= (unsigned long long)V.listper * (unsigned long long)V.nvec;
+      const size_t n = (size_t)V.nvec * (size_t)M.ncols;
+      if( !list )
       {
-         int64_t len = 0, beg = 0;
-         int32_t v = 0;
-         if( c0 + (uint32_t)t < n )
+         for( size_t flat = blockIdx.x * (size_t)SAP_BLOCK + t; flat < n; flat += (size_t)gridDim.x * SAP_BLOCK )
          {
-            const int2 e = V.touched[c0 + (uint32_t)t];
-            const size_t flat = (size_t)e.y * (size_t)M.ncols + (size_t)e.x;
-            if( V.chgtag[flat] == round && V.vcutoff[unitOfCol(M, e.y, e.x)] == 0 )
-            {
-               beg = M.colptr[e.x];
-               len = M.colptr[e.x + 1] - beg;
-               v = e.y;
-            }
+            if( V.chgtag[flat] != round )
+               continue;
+            const int32_t v = (int32_t)(flat / (size_t)M.ncols);
+            const int32_t j = (int32_t)(flat - (size_t)v * (size_t)M.ncols);
+            if( V.vcutoff[unitOfCol(M, v, j)] == 0 )
+               markColumn(M, V, j, v, next, anymarked);
          }
+      }
+      else
+      {
+         // the changed columns are collected in LDS and their rows listed SAP_BLOCK columns at
+         // a time (workgroup-uniform: nfound is read between barriers)
+         const unsigned nb = gridDim.x < SAP_MARK_BLOCKS ? gridDim.x : SAP_MARK_BLOCKS;
          if( t == 0 )
-            soff[0] = 0;
-         soff[t + 1] = len;
-         sbeg[t] = beg;
-         svec[t] = v;
+            nfound = 0;
          __syncthreads();
-         for( int d = 1; d < SAP_BLOCK; d <<= 1 )
+         for( size_t c0 = blockIdx.x * (size_t)SAP_MARK_FLATS; blockIdx.x < nb; c0 += (size_t)nb * SAP_MARK_FLATS )
          {
-            const int64_t add = t >= d ? soff[t + 1 - d] : 0;
+            const bool end = c0 >= n;
+            if( !end )
+#pragma unroll
+               for( int k = 0; k < SAP_MARK_FLATS / SAP_BLOCK; ++k )
+               {
+                  const size_t flat = c0 + (size_t)k * SAP_BLOCK + (size_t)t;
+                  if( flat < n && V.chgtag[flat] == round )
+                     found[atomicAdd(&nfound, 1u)] = (uint32_t)flat;   // nvec * ncols < 2^32
+               }
             __syncthreads();
-            soff[t + 1] += add;
-            __syncthreads();
-         }
-         const int64_t total = soff[SAP_BLOCK];
-         // passes of SAP_BLOCK rows (workgroup-uniform: total is read from LDS), appended per
-         // workgroup
-         for( int64_t f0 = 0; f0 < total; f0 += SAP_BLOCK )
-         {
-            const int64_t f = f0 + t;
-            bool fresh = false;
-            int bin = 0;
-            int2 item = make_int2(0, 0);
-            if( f < total )
+            uint32_t have = nfound;
+            while( have >= SAP_BLOCK || (end && have > 0) )
             {
-               // the entry of row f: the largest k with soff[k] <= f, which has soff[k + 1] > f
-               int lo = 0, hi = SAP_BLOCK - 1;
-               while( lo < hi )
+               const uint32_t take = have < SAP_BLOCK ? have : SAP_BLOCK;
+               int64_t len = 0, beg = 0;
+               int32_t v = 0;
+               if( (uint32_t)t < take )
                {
-                  const int mid = (lo + hi + 1) >> 1;
-                  if( soff[mid] <= f )
-                     lo = mid;
-                  else
-                     hi = mid - 1;
+                  const uint32_t flat = found[have - 1 - (uint32_t)t];
+                  v = (int32_t)(flat / (uint32_t)M.ncols);
+                  const int32_t j = (int32_t)(flat - (uint32_t)v * (uint32_t)M.ncols);
+                  if( V.vcutoff[unitOfCol(M, v, j)] == 0 )
+                  {
+                     beg = M.colptr[j];
+                     len = M.colptr[j + 1] - beg;
+                  }
                }
-               const int32_t rv = svec[lo];
-               const int32_t row = M.rowidx[sbeg[lo] + (f - soff[lo])];
-               const size_t rflat = (size_t)rv * (size_t)M.nrows + (size_t)row;
-               if( !rowRedundant(V, rflat) )
-               {
-                  if( V.vpend[rv] != next )
-                     V.vpend[rv] = next;   // every writer of this round stores the same value
-                  fresh = atomicMax(&V.rowmark[rflat], next) < next;
-                  bin = M.rowbin[row];
-                  item = make_int2(row, rv);
-               }
+               blockMark(M, V, S, beg, len, v, next, true, anymarked);
+               have -= take;
             }
-            blockAppendRows(st, V.wl[npar], npar, fresh, bin, item, scnt, sbase);
+            if( end )
+               break;
+            __syncthreads();   // every thread has read nfound
+            if( t == 0 )
+               nfound = have;
+            __syncthreads();
          }
-         __syncthreads();   // soff, sbeg and svec are rewritten by the next chunk
       }
    }
-   if( __ballot(anymarked) != 0 && ((int)threadIdx.x & (SAP_WAVE - 1)) == 0 && st->anymark[npar] == 0 )
-      st->anymark[npar] = 1;
+   if( V.dense && blockIdx.x == 0 && t == 0 )
+      st->listed[next & 1] = list ? 1 : 0;
+   if( __ballot(anymarked) != 0 && (t & (SAP_WAVE - 1)) == 0 && st->anymark[next & 1] == 0 )
+      st->anymark[next & 1] = 1;
 }
 
-__global__ __launch_bounds__(SAP_BLOCK) void k_mark(Mat M, Vec V)
+__global__ __launch_bounds__(SAP_BLOCK, 8) void k_mark(Mat M, Vec V)
 {
-   Status* st = V.st;
-   if( !(st->done || (V.single && st->cutoff)) )
-      markRound(M, V);
+   markRound(M, V);
 }
 
 // reason recording, after the column step: every logged candidate whose key won its column's
@@ -2846,9 +3080,12 @@ template <bool R>
 __global__ __launch_bounds__(SAP_BLOCK) void k_ranged(Mat M, Vec V, Params P)
 {
    Status* st = V.st;
-   if( st->done )
+   const RoundView view = roundView(V);
+   if( view.done )
       return;
-   const int32_t round = st->round;
+   const int32_t round = view.round;
+   Vec W = V;   // candidates join the touched list when the round's sweep keeps it (k_sweep)
+   W.dense = view.listed ? 0 : 1;
    if( V.dense )
    {
       const bool all = st->firstall && st->rlocal == 1;
@@ -2860,7 +3097,7 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_ranged(Mat M, Vec V, Params P)
          const int32_t row = M.rlist[i - (size_t)v * per];
          const size_t rflat = (size_t)v * (size_t)M.nrows + (size_t)row;
          if( (all || V.rowmark[rflat] == round) && !rowRedundant(V, rflat) && (R || !V.vcutoff[unitOfRow(M, v, row)]) )
-            rangedRow<R>(M, V, P, v, row);
+            rangedRow<R>(M, W, P, v, row);
       }
    }
    else
@@ -2868,14 +3105,14 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_ranged(Mat M, Vec V, Params P)
       const int flag = rangedRows(M, P) == M.nranged ? 2 : 4;
       for( int b = 0; b < SAP_NBINS; ++b )
       {
-         const uint32_t n = st->wlcount[round & 1][b];
+         const uint32_t n = st->wlcount[round & 1][b].n;
          const int2* wl = V.wl[round & 1][b];
          for( uint32_t i = blockIdx.x * SAP_BLOCK + threadIdx.x; i < n; i += gridDim.x * SAP_BLOCK )
          {
             const int2 it = wl[i];
             const size_t rflat = (size_t)it.y * (size_t)M.nrows + (size_t)it.x;
             if( (M.rowflags[it.x] & flag) && !rowRedundant(V, rflat) && (R || !V.vcutoff[unitOfRow(M, it.y, it.x)]) )
-               rangedRow<R>(M, V, P, it.y, it.x);
+               rangedRow<R>(M, W, P, it.y, it.x);
          }
       }
    }
@@ -2908,9 +3145,10 @@ __device__ __forceinline__ void roundAdvance(const Vec& V, int32_t maxrounds)
    st->rlocal += 1;
    st->clogn = 0;
    st->anymark[(r + 1) & 1] = 0;
+   st->listovf[(r + 1) & 1] = 0;
    for( int b = 0; b < SAP_NBINS; ++b )
-      st->wlcount[(r + 1) & 1][b] = 0;
-   st->touched = 0;
+      st->wlcount[(r + 1) & 1][b].n = 0;
+   st->touched.n = 0;
 }
 
 __global__ __launch_bounds__(SAP_STAT_SLOTS) void k_round_begin(Vec V, int32_t maxrounds)
@@ -2955,7 +3193,12 @@ __global__ void k_call_reset(Vec V, size_t nclear, int32_t nvec, int32_t firstal
       st->rgenm1 = gen - 1;
       st->anymark[0] = 0;
       st->anymark[1] = 0;
-      st->touched = 0;
+      st->listed[0] = 0;
+      st->listed[1] = 0;
+      st->listovf[0] = 0;
+      st->listovf[1] = 0;
+      st->chgbase = 0;
+      st->touched.n = 0;
       st->rows_swept = 0;
       st->nnz_swept = 0;
       st->nchg = 0;
@@ -2967,8 +3210,8 @@ __global__ void k_call_reset(Vec V, size_t nclear, int32_t nvec, int32_t firstal
       st->clogovf = 0;
       for( int b = 0; b < SAP_NBINS; ++b )
       {
-         st->wlcount[0][b] = 0;
-         st->wlcount[1][b] = 0;
+         st->wlcount[0][b].n = 0;
+         st->wlcount[1][b].n = 0;
       }
    }
    if( gi < SAP_STAT_SLOTS )
@@ -3005,43 +3248,7 @@ __global__ void k_init_all(Mat M, Vec V, int32_t bin, int32_t nvec)
    for( size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x; v < (size_t)nvec; v += (size_t)gridDim.x * blockDim.x )
       V.vpend[v] = st->round + 1;
    if( blockIdx.x == 0 && threadIdx.x == 0 )
-      st->wlcount[par][bin] = (uint32_t)tot;
-}
-
-// initial marks / worklists from overlay columns (base bounds already a fixpoint)
-__global__ void k_init_overlay(Mat M, Vec V, const int64_t* ovptr, const int32_t* ovcol, int32_t nvec)
-{
-   Status* st = V.st;
-   const int32_t first = st->round + 1;
-   const int par = first & 1;
-   bool any = false;
-   for( int32_t v = blockIdx.y; v < nvec; v += gridDim.y )
-   {
-      for( int64_t q = ovptr[v] + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < ovptr[v + 1];
-           q += (int64_t)gridDim.x * blockDim.x )
-      {
-         const int32_t j = ovcol[q];
-         for( int64_t r = M.colptr[j]; r < M.colptr[j + 1]; ++r )
-         {
-            const int32_t row = M.rowidx[r];
-            const size_t rflat = (size_t)v * (size_t)M.nrows + (size_t)row;
-            if( V.vpend[v] != first )
-               V.vpend[v] = first;
-            if( V.dense )
-            {
-               V.rowmark[rflat] = first;
-               any = true;
-            }
-            else
-            {
-               const bool fresh = atomicMax(&V.rowmark[rflat], first) < first;
-               waveAppendRow(st, V.wl[par], par, fresh, M.rowbin[row], make_int2(row, v));
-            }
-         }
-      }
-   }
-   if( __ballot(any) != 0 && ((int)threadIdx.x & (SAP_WAVE - 1)) == 0 )
-      st->anymark[par] = 1;
+      st->wlcount[par][bin].n = (uint32_t)tot;
 }
 
 // ---- slots: admission, step control, collection (vector indices through a slot list) ----
@@ -3143,21 +3350,15 @@ __device__ __forceinline__ void slotMarkRow(const Mat& M, const Vec& V, Status* 
 
 // marks for the first round of the admitted slots: the rows of the overlay columns (base is a
 // fixpoint), or every row (grid: rows per slot in x, slots in y).  The overlay entries of all
-// slots (ovptr[0] = 0 .. ovptr[n]) are taken SAP_BLOCK at a time over a one-dimensional grid,
-// each thread finding its slot by binary search in ovptr, and the (column, row) pairs of a
-// chunk are numbered across the workgroup (a scan of the column lengths in LDS).  So a
-// wavefront appends up to 64 rows to the worklists at once, also when every slot has a single
-// overlay column (probing): a workgroup or thread per slot or column would leave most lanes
-// idle and make one append per row, and the appends of all slots contend on the few worklist
-// counters.  Launched with SAP_BLOCK threads.
+// slots (ovptr[0] = 0 .. ovptr[n]) are taken `chunk` at a time over a one-dimensional grid,
+// each thread finding its slot by binary search in ovptr, and their rows are marked and listed
+// by the workgroup (blockMark).  listed: dense mode's flag of this round after the call (1
+// also lists, 0 tags alone suffice to mark; -1 as 1, but leaves the flag, which an earlier
+// marking for the same round may have cleared).  Launched with SAP_BLOCK threads.
 __global__ void __launch_bounds__(SAP_BLOCK) k_slot_mark(Mat M, Vec V, const int32_t* slots, int32_t n,
-   const int64_t* ovptr, const int32_t* ovcol, int32_t allrows, int32_t chunk)
+   const int64_t* ovptr, const int32_t* ovcol, int32_t allrows, int32_t chunk, int32_t listed)
 {
-   __shared__ int64_t soff[SAP_BLOCK + 1];   // soff[k]: pairs of the chunk's columns before column k
-   __shared__ int64_t sbeg[SAP_BLOCK];       // colptr of column k
-   __shared__ int32_t svec[SAP_BLOCK];       // vector of column k
-   __shared__ uint32_t scnt[SAP_NBINS];      // fresh rows of one pass per length bin
-   __shared__ uint32_t sbase[SAP_NBINS];     // their first worklist position
+   __shared__ MarkShared S;
    Status* st = V.st;
    const int32_t first = st->round + 1;
    const int par = first & 1;
@@ -3199,64 +3400,15 @@ __global__ void __launch_bounds__(SAP_BLOCK) k_slot_mark(Mat M, Vec V, const int
             beg = M.colptr[j];
             len = M.colptr[j + 1] - beg;
          }
-         if( t == 0 )
-            soff[0] = 0;
-         soff[t + 1] = len;
-         sbeg[t] = beg;
-         svec[t] = v;
-         __syncthreads();
-         for( int d = 1; d < SAP_BLOCK; d <<= 1 )
-         {
-            const int64_t add = t >= d ? soff[t + 1 - d] : 0;
-            __syncthreads();
-            soff[t + 1] += add;
-            __syncthreads();
-         }
-         const int64_t total = soff[SAP_BLOCK];
-         // passes of SAP_BLOCK pairs (workgroup-uniform: total is read from LDS); the fresh
-         // rows of a pass are counted per length bin in LDS and appended with one global
-         // atomic per bin and workgroup
-         for( int64_t f0 = 0; f0 < total; f0 += SAP_BLOCK )
-         {
-            const int64_t f = f0 + t;
-            bool fresh = false;
-            int bin = 0;
-            int2 item = make_int2(0, 0);
-            if( f < total )
-            {
-               // the column of pair f: the largest k with soff[k] <= f (soff[0] = 0 <= f; such
-               // a k has soff[k + 1] > f, so a column with rows)
-               int lo = 0, hi = SAP_BLOCK - 1;
-               while( lo < hi )
-               {
-                  const int mid = (lo + hi + 1) >> 1;
-                  if( soff[mid] <= f )
-                     lo = mid;
-                  else
-                     hi = mid - 1;
-               }
-               const int32_t rv = svec[lo];
-               const int32_t row = M.rowidx[sbeg[lo] + (f - soff[lo])];
-               const size_t rflat = (size_t)rv * (size_t)M.nrows + (size_t)row;
-               if( V.vpend[rv] != first )
-                  V.vpend[rv] = first;
-               if( V.dense )
-               {
-                  V.rowmark[rflat] = first;
-                  any = true;
-               }
-               else
-               {
-                  fresh = atomicMax(&V.rowmark[rflat], first) < first;
-                  bin = M.rowbin[row];
-                  item = make_int2(row, rv);
-               }
-            }
-            blockAppendRows(st, V.wl[par], par, fresh, bin, item, scnt, sbase);
-         }
-         __syncthreads();   // soff, sbeg and svec are rewritten by the next chunk
+         if( !V.dense || listed != 0 )
+            blockMark(M, V, S, beg, len, v, first, false, any);
+         else
+            for( int64_t q = beg; q < beg + len; ++q )
+               slotMarkRow(M, V, st, v, M.rowidx[q], first, par, any);
       }
    }
+   if( V.dense && blockIdx.x == 0 && blockIdx.y == 0 && t == 0 && listed >= 0 )
+      st->listed[par] = listed;
    if( __ballot(any) != 0 && ((int)threadIdx.x & (SAP_WAVE - 1)) == 0 )
       st->anymark[par] = 1;
 }
@@ -3281,6 +3433,7 @@ __global__ void k_step_begin(Vec V)
       st->cutoff = 0;
       st->rlocal = 0;
       st->firstall = 0;
+      st->chgbase = 0;
       st->sweep_ticks = 0;
       st->sweep_count = 0;
    }
@@ -3430,23 +3583,6 @@ __global__ void k_probe_pairs(Vec V, int64_t ncols, const int32_t* pcol, int32_t
    }
 }
 
-// bounds of all vectors from a base vector plus overlays
-__global__ void k_broadcast_base(double2* bnd, const double2* base, int64_t ncols, int32_t nvec)
-{
-   const size_t tot = (size_t)nvec * (size_t)ncols;
-   for( size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < tot; i += (size_t)gridDim.x * blockDim.x )
-      bnd[i] = base[i % (size_t)ncols];
-}
-
-__global__ void k_apply_overlay(double2* bnd, int64_t ncols, const int64_t* ovptr, const int32_t* ovcol,
-   const double* ovlb, const double* ovub, int32_t nvec)
-{
-   for( int32_t v = blockIdx.y; v < nvec; v += gridDim.y )
-      for( int64_t q = ovptr[v] + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < ovptr[v + 1];
-           q += (int64_t)gridDim.x * blockDim.x )
-         bnd[(size_t)v * (size_t)ncols + (size_t)ovcol[q]] = make_double2(ovlb[q], ovub[q]);
-}
-
 __global__ void k_fill_i64(long long* p, long long val, size_t n)
 {
    for( size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x )
@@ -3584,7 +3720,9 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_row_activities(Mat M, Params P, c
 // columns and SAP_NOALLOC_MAXROWS rows: 56 B per column, 5 B per row, 256-byte aligned pieces.
 #define SAP_NOALLOC_MAXCOLS ((int64_t)1 << 20)
 #define SAP_NOALLOC_MAXROWS ((int64_t)1 << 20)
-#define SAP_NOALLOC_BYTES ((size_t)SAP_NOALLOC_MAXCOLS * 56 + (size_t)SAP_NOALLOC_MAXROWS * 5 + ((size_t)1 << 16))
+#define SAP_NOALLOC_LIST ((uint32_t)1 << 15)   // entries of each worklist
+#define SAP_NOALLOC_BYTES ((size_t)SAP_NOALLOC_MAXCOLS * 56 + (size_t)SAP_NOALLOC_MAXROWS * 5 + \
+   (2 * SAP_NBINS + 1) * 8 * (size_t)SAP_NOALLOC_LIST + ((size_t)1 << 16))
 static __device__ __align__(256) unsigned char g_noalloc_scratch[SAP_NOALLOC_BYTES];
 
 struct sap_context
@@ -4068,7 +4206,7 @@ int sap_context_create(int32_t device, sap_context** out)
    HIPCHK(hipGetSymbolAddress((void**)&c->scratch, HIP_SYMBOL(g_noalloc_scratch)));
    int ncu = 0, per = 0;
    if( hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess
-      && hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_sweep<false>, SAP_BLOCK, 0) == hipSuccess && ncu > 0
+      && hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_sweep<false, true>, SAP_BLOCK, 0) == hipSuccess && ncu > 0
       && per > 0 )
       c->resident = ncu * per;
    *out = c;
@@ -4768,6 +4906,25 @@ static void boundsRelease(sap_bounds* b)
 // and vector) stays small against the row sweep itself
 #define SAP_DENSE_LIMIT ((size_t)1 << 24)
 
+// worklist room and, in dense mode, the changed columns up to which a round's rows are listed.
+// Each dense list holds at most SAP_LIST_ROWS rows (18 lists, 8 B a row); the columns are as
+// many as mark a quarter of the rows.  Measured on the mixed 1M x 1M instance: a listed sweep of
+// a row costs about twice its share of a full tile sweep.
+#define SAP_LIST_ROWS ((uint32_t)1 << 17)
+#define SAP_LIST_COLS ((uint32_t)1 << 16)
+
+static void listLimits(const sap_matrix* m, Vec& V)
+{
+   V.listcap = V.touchcap = UINT32_MAX;
+   V.listper = 0;
+   if( !V.dense )
+      return;
+   V.listcap = SAP_LIST_ROWS;
+   V.touchcap = SAP_LIST_COLS;
+   const double deg = m->ncols > 0 ? (double)m->nnz / (double)m->ncols : 0.0;
+   V.listper = (uint32_t)std::max(1.0, std::min(1e9, (double)m->nrows / 64.0 / std::max(deg, 1.0)));
+}
+
 int sap_bounds_create(sap_matrix* m, int32_t nvec, sap_bounds** out)
 {
    return sap_bounds_create_mode(m, nvec, SAP_MODE_AUTO, out);
@@ -4832,13 +4989,11 @@ int sap_bounds_create_mode(sap_matrix* m, int32_t nvec, int32_t mode, sap_bounds
    BALLOC(b->slotidx2, nvec);
    BALLOC(b->outoff, (size_t)nvec + 1);
    BALLOC(b->ident, nvec);
-   if( !V.dense )
-   {
-      for( int p = 0; p < 2; ++p )
-         for( int q = 0; q < SAP_NBINS; ++q )
-            BALLOC(V.wl[p][q], (size_t)nvec * (size_t)(m->binstart[q + 1] - m->binstart[q]));
-      BALLOC(V.touched, NC);
-   }
+   listLimits(m, V);
+   for( int p = 0; p < 2; ++p )
+      for( int q = 0; q < SAP_NBINS; ++q )
+         BALLOC(V.wl[p][q], std::min((size_t)nvec * (size_t)(m->binstart[q + 1] - m->binstart[q]), (size_t)V.listcap));
+   BALLOC(V.touched, std::min(NC, (size_t)V.touchcap));
    BALLOC(b->dstatus, 1);
    BALLOC(b->stage, 2 * (size_t)m->ncols);
 #undef BALLOC
@@ -4988,6 +5143,15 @@ static Layout makeLayout(const sap_bounds* b)
    return L;
 }
 
+// workgroups of a sweep launch: those of the layout, and enough to share out a listed round's
+// bins one each (listShare)
+#define SAP_LISTGRID 64
+
+static int sweepGrid(const Layout& L)
+{
+   return L.blockstart[SAP_NKINDS] > 0 ? std::max(L.blockstart[SAP_NKINDS], SAP_LISTGRID) : 0;
+}
+
 // host twin of foldStamps, on a status read back from the device
 static void hostFoldStamps(Status* h)
 {
@@ -5041,7 +5205,7 @@ static void enqueueRound(sap_bounds* b, const Mat& M, const Params& P, const Lay
    hipEvent_t e1, bool begun = false)
 {
    sap_matrix* m = b->mat;
-   const int nsweep = L.blockstart[SAP_NKINDS];
+   const int nsweep = sweepGrid(L);
    const unsigned colgrid = gridFor((size_t)b->V.nvec * (size_t)m->ncols, 4096);
    if( !begun )
       k_round_begin<<<1, SAP_STAT_SLOTS, 0, s>>>(b->V, P.maxrounds);
@@ -5053,9 +5217,11 @@ static void enqueueRound(sap_bounds* b, const Mat& M, const Params& P, const Lay
    if( e0 != NULL )
       (void)hipEventRecord(e0, s);
    if( nsweep > 0 && b->V.reasons )
-      k_sweep<true><<<nsweep, SAP_BLOCK, 0, s>>>(M, b->V, P, L);
+      k_sweep<true, true><<<nsweep, SAP_BLOCK, 0, s>>>(M, b->V, P, L);
+   else if( nsweep > 0 && b->V.dense )
+      k_sweep<false, true><<<nsweep, SAP_BLOCK, 0, s>>>(M, b->V, P, L);
    else if( nsweep > 0 )
-      k_sweep<false><<<nsweep, SAP_BLOCK, 0, s>>>(M, b->V, P, L);
+      k_sweep<false, false><<<nsweep, SAP_BLOCK, 0, s>>>(M, b->V, P, L);
    if( e1 != NULL )
       (void)hipEventRecord(e1, s);
    k_columns<<<colgrid, SAP_BLOCK, 0, s>>>(M, b->V, P);
@@ -5833,6 +5999,12 @@ static unsigned slotMarkBlocks(int64_t nov)
    return (unsigned)(g < 1 ? 1 : (g > 8192 ? 8192 : g));
 }
 
+// few enough overlay columns for the call's vectors that their rows are listed (dense mode)
+static bool listsOverlay(const sap_bounds* b, int64_t nov)
+{
+   return nov <= (int64_t)b->V.listper * (int64_t)b->V.nvec;
+}
+
 static dim3 slotGrid(size_t perslot, int32_t n)
 {
    return dim3(gridFor(perslot, 64), (unsigned)std::min<int32_t>(n > 0 ? n : 1, 65535));
@@ -5906,7 +6078,7 @@ static int admitSlots(sap_bounds* b, int32_t n, const int32_t* hslots, const int
          b->ovcol, b->ovlb, b->ovub);
    if( allrows || nov > 0 )
       k_slot_mark<<<allrows ? slotGrid((size_t)m->nrows, n) : dim3(slotMarkBlocks(nov)), SAP_BLOCK, 0, s>>>(M, b->V,
-         dslots, n, b->ovptr, b->ovcol, allrows, slotMarkChunk(nov));
+         dslots, n, b->ovptr, b->ovcol, allrows, slotMarkChunk(nov), (!allrows && listsOverlay(b, nov)) ? -1 : 0);
    HIPCHK(hipGetLastError());
    return SAP_OKAY;
 }
@@ -6122,7 +6294,7 @@ static int batchCall(sap_bounds* b, const sap_params* params, int32_t nvec, cons
             nvec, b->ovptr, b->ovcol, b->ovlb, b->ovub);
       if( fromfix && nov > 0 )
          k_slot_mark<<<dim3(slotMarkBlocks(nov)), SAP_BLOCK, 0, s>>>(toMat(m), b->V, b->ident, nvec,
-            b->ovptr, b->ovcol, 0, slotMarkChunk(nov));
+            b->ovptr, b->ovcol, 0, slotMarkChunk(nov), listsOverlay(b, nov) ? 1 : 0);
       rc = hipToRc(hipGetLastError());
    }
    if( rc == SAP_OKAY && !fromfix && !b->V.dense )
@@ -6870,6 +7042,13 @@ int sap_propagate_device_noalloc(sap_matrix* m, const sap_params* params, double
    V.vstart = (int32_t*)take(4);
    V.vpend = (int32_t*)take(4);
    V.vlogn = (int32_t*)take(4);
+   listLimits(m, V);
+   V.listcap = SAP_NOALLOC_LIST;
+   V.touchcap = SAP_NOALLOC_LIST;
+   for( int p = 0; p < 2; ++p )
+      for( int q = 0; q < SAP_NBINS; ++q )
+         V.wl[p][q] = (int2*)take(sizeof(int2) * SAP_NOALLOC_LIST);
+   V.touched = (int2*)take(sizeof(int2) * SAP_NOALLOC_LIST);
    b.dstatus = (Status*)take(sizeof(Status));
    V.st = b.dstatus;
    if( (size_t)(next - c->scratch) > SAP_NOALLOC_BYTES )

@@ -1,0 +1,72 @@
+"""Rounds swept from row lists in dense bound sets, at the sizes where the lists end: one column
+of very high degree is fixed, so that few changed columns mark many rows (more than a row list
+holds) and these touch many columns (more than the touched list holds).  Against the oracle's
+Jacobi twin: bit-exact bounds, verdicts, rounds and counts."""
+import numpy as np
+import pytest
+
+import scip_amd as sa
+from oracle import oracle as orc
+from tests.test_zz_no_alloc import DeviceArray
+
+pytestmark = pytest.mark.gpu
+
+
+def star(n, force):
+    """x0 + y_i + y_(i+1) <= 1 over binaries for i = 1..n, then (force) the row x0 >= 1: its round
+    changes one column, whose n rows then fix every y."""
+    rows = n + (1 if force else 0)
+    rowptr = np.concatenate([3 * np.arange(n + 1), [3 * n + 1] if force else []]).astype(np.int64)
+    i = np.arange(1, n + 1)
+    colidx = np.stack([np.zeros(n, np.int64), i, i + 1], 1).reshape(-1)
+    colidx = np.concatenate([colidx, [0]] if force else [colidx]).astype(np.int32)
+    lhs, rhs = np.full(rows, -1e20), np.full(rows, 1.0)
+    if force:
+        lhs[n], rhs[n] = 1.0, 1e20
+    return sa.Instance(rowptr=rowptr, colidx=colidx, vals=np.ones(len(colidx)), lhs=lhs, rhs=rhs,
+                       integral=np.ones(n + 2, dtype=np.uint8), lb=np.zeros(n + 2), ub=np.ones(n + 2))
+
+
+# rows of one length bin and touched columns: within every list; beyond the no-allocation
+# entry point's lists (2^15); beyond the touched list (2^16); beyond a row list (2^17)
+@pytest.mark.parametrize("n", [32_700, 33_000, 70_000, 131_000, 135_000])
+def test_lists_end(gpu_ctx, n):
+    print(f"[case] lists n={n}", flush=True)
+    inst = star(n, force=True)
+    ol, ou, orr = orc.propagate_jacobi(orc.OMatrix.from_instance(inst), inst.lb, inst.ub)
+    assert not orr["cutoff"] and orr["rounds"] == 3 and orr["nchgbds"] == n + 2
+    mat = sa.Matrix(gpu_ctx, inst)
+    lb, ub, st = mat.propagate()
+    assert np.array_equal(lb, ol) and np.array_equal(ub, ou)
+    assert (st["rounds"], st["nchgbds"], st["rows_swept"]) == (orr["rounds"], orr["nchgbds"], orr["rows_swept"])
+    dl, du = DeviceArray(inst.lb), DeviceArray(inst.ub)
+    st = mat.propagate_device_noalloc(dl.data_ptr(), du.data_ptr())
+    assert np.array_equal(dl.numpy(), ol) and np.array_equal(du.numpy(), ou)
+    assert (st["rounds"], st["nchgbds"], st["rows_swept"]) == (orr["rounds"], orr["nchgbds"], orr["rows_swept"])
+    dl.free()
+    du.free()
+    mat.close()
+
+
+@pytest.mark.parametrize("n", [70_000, 135_000])
+def test_lists_end_from_overlays(gpu_ctx, n):
+    # the same rows marked by a node's overlay, next to a node with a single marked row pair and
+    # one that is cut off, in one dense set; then again on the same set
+    print(f"[case] lists from overlays n={n}", flush=True)
+    inst = star(n, force=False)
+    mat = sa.Matrix(gpu_ctx, inst)
+    base = sa.Bounds(mat, 1)
+    base.upload(inst.lb, inst.ub)
+    nodes = sa.Bounds(mat, 3, sa.SAP_MODE_DENSE)
+    p = sa.default_params(flags=sa.SAP_FLAG_BASE_IS_FIXPOINT)
+    for _ in range(2):
+        out = nodes.propagate_nodes(base, 0, [0, 1, 2, 4], [0, 5, 7, 8], [1.0] * 4, [1.0] * 4, params=p,
+                                    chgcap=2 * n + 64)
+        assert out["result"].tolist() == [sa.SAP_REDUCEDDOM, sa.SAP_REDUCEDDOM, sa.SAP_CUTOFF]
+        assert out["rounds"][:2].tolist() == [2, 2]
+        a, b, c = out["chgptr"][1:].tolist()
+        assert np.array_equal(out["chgcol"][:a], np.arange(1, n + 2)) and np.all(out["chgub"][:a] == 0.0)
+        assert out["chgcol"][a:b].tolist() == [0, 4, 6] and np.all(out["chgub"][a:b] == 0.0) and b == c
+    nodes.close()
+    base.close()
+    mat.close()
