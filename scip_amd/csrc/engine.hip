@@ -2669,7 +2669,7 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
    {
       const unsigned used = gridDim.x < SAP_STAT_SLOTS ? gridDim.x : SAP_STAT_SLOTS;
       const unsigned scale = used > SAP_CHG_SAMPLE ? used / SAP_CHG_SAMPLE : 1;
-      list = changed * scale <= (unsigned long long)V.listper * (unsigned long long)V.nvec;
+      list = V.listper > 0 && changed * scale <= (unsigned long long)V.listper * (unsigned long long)V.nvec;
       const size_t n = (size_t)V.nvec * (size_t)M.ncols;
       if( !list )
       {
@@ -4907,11 +4907,17 @@ static void boundsRelease(sap_bounds* b)
 #define SAP_DENSE_LIMIT ((size_t)1 << 24)
 
 // worklist room and, in dense mode, the changed columns up to which a round's rows are listed.
-// Each dense list holds at most SAP_LIST_ROWS rows (18 lists, 8 B a row); the columns are as
-// many as mark a quarter of the rows.  Measured on the mixed 1M x 1M instance: a listed sweep of
-// a row costs about twice its share of a full tile sweep.
+// Each dense list holds at most SAP_LIST_ROWS rows (18 lists, 8 B a row).
+//   - 1/64 of the rows marked: on the mixed 1M x 1M instance rounds 5-7 (11,807, 324 and 11 rows)
+//     sweep in 57 / 22 / 12 us listed against 79 / 45 / 29 us scanned, and 1/4 listed its round 4,
+//     which then took 214 + 42 us to sweep and to list for against 173 + 10 us;
+//   - sets of few tiles are not listed: a scan visits each wavefront's one tile, while the lists
+//     add their own steps (2,875 x 4,443, 5 rounds: 266 us listed, 254 us scanned).
+// 200 strong-branching children of 20,011 rows take 310 us (555-597 us scanned), a node of
+// 148,409 rows among 31 a third of what it took.
 #define SAP_LIST_ROWS ((uint32_t)1 << 17)
 #define SAP_LIST_COLS ((uint32_t)1 << 16)
+#define SAP_LIST_TILES 2048
 
 static void listLimits(const sap_matrix* m, Vec& V)
 {
@@ -4921,6 +4927,8 @@ static void listLimits(const sap_matrix* m, Vec& V)
       return;
    V.listcap = SAP_LIST_ROWS;
    V.touchcap = SAP_LIST_COLS;
+   if( (int64_t)V.nvec * m->ntiles <= SAP_LIST_TILES )
+      return;
    const double deg = m->ncols > 0 ? (double)m->nnz / (double)m->ncols : 0.0;
    V.listper = (uint32_t)std::max(1.0, std::min(1e9, (double)m->nrows / 64.0 / std::max(deg, 1.0)));
 }
@@ -6002,7 +6010,7 @@ static unsigned slotMarkBlocks(int64_t nov)
 // few enough overlay columns for the call's vectors that their rows are listed (dense mode)
 static bool listsOverlay(const sap_bounds* b, int64_t nov)
 {
-   return nov <= (int64_t)b->V.listper * (int64_t)b->V.nvec;
+   return b->V.listper > 0 && nov <= (int64_t)b->V.listper * (int64_t)b->V.nvec;
 }
 
 static dim3 slotGrid(size_t perslot, int32_t n)
