@@ -3657,6 +3657,32 @@ __global__ void k_deinterleave(const double2* src, double* lb, double* ub, int64
    }
 }
 
+// the outcome of a call on vector 0, written to mapped host memory after every round group once
+// the call has ended (its done flag, or the stop test the host applies after the group): the
+// bounds (lb NULL: not asked for), and the first histmax entries of the reason history as 32-bit
+// words (hist NULL: none)
+__global__ void k_land(Vec V, int64_t ncols, int32_t maxrounds, double* lb, double* ub, uint32_t* hist, uint32_t histmax)
+{
+   const Status* st = V.st;
+   if( !st->done && !stopsNext(*st, V.dense != 0, maxrounds) )
+      return;
+   const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+   if( hist != NULL )
+   {
+      const int64_t n = (int64_t)(st->histn < histmax ? st->histn : histmax) * (int64_t)(sizeof(HistRec) / 4);
+      for( int64_t i = i0; i < n; i += step )
+         hist[i] = ((const uint32_t*)V.hist)[i];
+   }
+   if( st->cutoff )
+      return;   // no bounds come back from an infeasible call
+   for( int64_t i = i0; i < ncols; i += step )
+   {
+      const double2 b = V.bnd[i];
+      lb[i] = b.x;
+      ub[i] = b.y;
+   }
+}
+
 // the memory floor of the row sweep: the sweep's own streams and gathers without its
 // arithmetic.  Lane i of the grid takes nonzeros 4i..4i+3 (the four positions of a lane of a
 // width-4 tile), reads them as one vector of column indices and two of values, so that a
@@ -3725,6 +3751,11 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_row_activities(Mat M, Params P, c
    (2 * SAP_NBINS + 1) * 8 * (size_t)SAP_NOALLOC_LIST + ((size_t)1 << 16))
 static __device__ __align__(256) unsigned char g_noalloc_scratch[SAP_NOALLOC_BYTES];
 
+// host bound arrays move in chunks of SAP_RING_COLS columns (512 KiB) through SAP_RING_SLOTS
+// pinned slots; arrays of at most one chunk move in one piece, with the call's own wait
+#define SAP_RING_COLS ((int64_t)32768)
+#define SAP_RING_SLOTS 8
+
 struct sap_context
 {
    int32_t device;
@@ -3739,6 +3770,13 @@ struct sap_context
    Status* hstatusd;  // ... written by a copy kernel through this device address
    unsigned char* scratch;   // this device's address of the no-allocation scratch array
    int32_t resident;         // sweep workgroups the device holds at once (0: unknown)
+   // pinned, mapped and coherent staging of host bound arrays (ensureRing), with its device
+   // address; busy: a kernel that reads it may be in flight
+   char* ring;
+   char* ringd;
+   size_t ringcap;
+   int32_t ringbusy;
+   hipEvent_t ringev[SAP_RING_SLOTS];
 };
 
 struct sap_matrix
@@ -4228,6 +4266,11 @@ int sap_context_free(sap_context* c)
    for( int i = 0; i < 4; ++i )
       (void)hipEventDestroy(c->ev[i]);
    (void)hipHostFree(c->hstatus);
+   if( c->ring != NULL )
+      (void)hipHostFree(c->ring);
+   for( int i = 0; i < SAP_RING_SLOTS; ++i )
+      if( c->ringev[i] != NULL )
+         (void)hipEventDestroy(c->ringev[i]);
    (void)hipStreamDestroy(c->cstream);
    (void)hipStreamDestroy(c->stream);
    free(c);
@@ -5060,26 +5103,223 @@ static void touchedVectors(sap_bounds* b, int32_t v)
       (*b->srcb)[(size_t)q] = NULL;
 }
 
+}   // extern "C"
+
+static int pinnedArea(size_t bytes, char** h, char** d);
+
+// pinned staging of at least `bytes` on context c; what is in it may be overwritten afterwards
+static int ensureRing(sap_context* c, size_t bytes)
+{
+   if( c->ringbusy || bytes > c->ringcap )
+   {
+      HIPCHK(hipStreamSynchronize(c->stream));
+      c->ringbusy = 0;
+   }
+   if( bytes <= c->ringcap )
+      return SAP_OKAY;
+   if( c->ring != NULL )
+      (void)hipHostFree(c->ring);
+   c->ring = c->ringd = NULL;
+   c->ringcap = 0;
+   RCCHK(pinnedArea(bytes, &c->ring, &c->ringd));
+   c->ringcap = bytes;
+   return SAP_OKAY;
+}
+
+// some element of x[0..n) is NaN (no early exit, so that it vectorises)
+static bool anyNan(const double* x, int64_t n)
+{
+   int bad = 0;
+   for( int64_t j = 0; j < n; ++j )
+      bad |= x[j] != x[j];
+   return bad != 0;
+}
+
+// helper threads of a host array's transfer: as many as can be started, at most `want`
+template <typename F>
+static void startThreads(std::vector<std::thread>& th, int want, F fn)
+{
+   const int hw = (int)std::thread::hardware_concurrency();
+   try
+   {
+      for( int t = 0; t < want && t < hw - 1; ++t )
+         th.emplace_back(fn);
+   }
+   catch( ... )
+   {
+      // the calling thread does what no helper takes
+   }
+}
+
+// vector v (all for v < 0) of b from host arrays, refused if they hold a NaN.  Up to
+// SAP_RING_COLS columns go through pinned staging and one kernel that reads it, with no wait
+// (two pageable copies waited 10-20 us each): the caller's later wait covers it.  With the
+// result landing by the call's own wait as well, sap_propagate on 2,000 x 5,000 went from 135 to
+// 87 us.  Longer arrays
+// are copied by the runtime, which reads pageable memory at the link's rate (25 us a MiB),
+// while helper threads look for NaNs.  room: staging the caller needs behind the arrays.
+static int uploadBounds(sap_bounds* b, int32_t v, const double* lb, const double* ub, size_t room = 0)
+{
+   sap_matrix* m = b->mat;
+   sap_context* c = m->ctx;
+   hipStream_t s = c->stream;
+   const int64_t nc = m->ncols;
+   const double *dl = b->stage, *du = b->stage + nc;
+   if( nc <= SAP_RING_COLS )
+   {
+      if( anyNan(lb, nc) || anyNan(ub, nc) )
+         return SAP_INVALIDDATA;
+      RCCHK(ensureRing(c, 16 * (size_t)nc + room));
+      if( nc > 0 )
+      {
+         memcpy(c->ring, lb, 8 * (size_t)nc);
+         memcpy(c->ring + 8 * (size_t)nc, ub, 8 * (size_t)nc);
+      }
+      dl = (const double*)c->ringd;
+      du = dl + nc;
+      c->ringbusy = 1;
+   }
+   else
+   {
+      const int64_t part = 8 * SAP_RING_COLS;
+      std::atomic<int64_t> next(0);
+      std::atomic<int> bad(0);
+      auto look = [&]() {
+         for( int64_t j = next.fetch_add(part); j < nc && !bad; j = next.fetch_add(part) )
+         {
+            const int64_t n = std::min(part, nc - j);
+            if( anyNan(lb + j, n) || anyNan(ub + j, n) )
+               bad = 1;
+         }
+      };
+      std::vector<std::thread> th;
+      startThreads(th, (int)std::min<int64_t>(3, nc / part), look);
+      hipError_t e = hipMemcpyAsync(b->stage, lb, sizeof(double) * (size_t)nc, hipMemcpyHostToDevice, s);
+      if( e == hipSuccess )
+         e = hipMemcpyAsync(b->stage + nc, ub, sizeof(double) * (size_t)nc, hipMemcpyHostToDevice, s);
+      look();
+      for( auto& x : th )
+         x.join();
+      if( e != hipSuccess || bad )
+         HIPCHK(hipStreamSynchronize(s));   // the caller's arrays are not read after the return
+      HIPCHK(e);
+      if( bad )
+         return SAP_INVALIDDATA;
+   }
+   const int32_t v0 = v < 0 ? 0 : v, v1 = v < 0 ? b->nvec : v + 1;
+   for( int32_t q = v0; q < v1; ++q )
+      k_interleave<<<gridFor((size_t)nc), SAP_BLOCK, 0, s>>>(b->V.bnd + (size_t)q * (size_t)nc, dl, du, nc);
+   HIPCHK(hipGetLastError());
+   touchedVectors(b, v);
+   return SAP_OKAY;
+}
+
+// (lb, ub) pairs of src as host arrays, handed out in chunks: take(j0, n, l, u) for columns
+// [j0, j0 + n), from several threads at once and in any order.  A kernel writes each chunk to a
+// pinned slot while helper threads copy the earlier ones out: copying 16 MB to pageable memory
+// through the runtime took 80 us a MiB, three quarters of it a memcpy with the device idle
+// (16 MB: 924 us, now 448 us; the kernel writes a 512 KiB chunk in 10 us).
+template <typename F>
+static int downloadBounds(sap_context* c, const double2* src, int64_t nc, F take)
+{
+   hipStream_t s = c->stream;
+   const int64_t cols = std::min(SAP_RING_COLS, std::max<int64_t>(nc, 1));
+   const int64_t nchunks = (nc + cols - 1) / cols;
+   const int64_t slots = std::min<int64_t>(SAP_RING_SLOTS, nchunks);
+   RCCHK(ensureRing(c, 16 * (size_t)cols * (size_t)std::max<int64_t>(slots, 1)));
+   for( int64_t q = 0; q < slots; ++q )
+      if( c->ringev[q] == NULL )
+         HIPCHK(hipEventCreateWithFlags(&c->ringev[q], hipEventDisableTiming));
+   std::atomic<int64_t> ready(0), next(0);
+   std::vector<std::atomic<int>> copied((size_t)nchunks);
+   for( auto& x : copied )
+      x = 0;
+   auto copyOut = [&](int64_t q) {
+      const double* l = (const double*)(c->ring + 16 * (size_t)cols * (size_t)(q % slots));
+      take(q * cols, std::min(cols, nc - q * cols), l, l + cols);
+      copied[(size_t)q].store(1, std::memory_order_release);
+   };
+   // ready counts the landed chunks; nchunks + 1 stops the helpers early (an error)
+   auto help = [&]() {
+      for( int64_t q = next.fetch_add(1); q < nchunks; q = next.fetch_add(1) )
+      {
+         while( ready.load(std::memory_order_acquire) <= q )
+            std::this_thread::yield();
+         if( ready.load(std::memory_order_acquire) > nchunks )
+            return;
+         copyOut(q);
+      }
+   };
+   auto launch = [&](int64_t q) -> hipError_t {
+      double* l = (double*)(c->ringd + 16 * (size_t)cols * (size_t)(q % slots));
+      const int64_t n = std::min(cols, nc - q * cols);
+      k_deinterleave<<<gridFor((size_t)n), SAP_BLOCK, 0, s>>>(src + q * cols, l, l + cols, n);
+      const hipError_t e = hipGetLastError();
+      return e != hipSuccess ? e : hipEventRecord(c->ringev[q % slots], s);
+   };
+   hipError_t e = hipSuccess;
+   for( int64_t q = 0; q < slots && e == hipSuccess; ++q )
+      e = launch(q);
+   std::vector<std::thread> th;
+   if( nchunks > 2 )
+      startThreads(th, (int)std::min<int64_t>(4, nchunks / 2), help);
+   // chunk q lands in its slot once chunk q - slots has been copied out of it; the loop only
+   // waits for that when no chunk is in flight
+   int64_t launched = slots;
+   auto refill = [&](int64_t upto) {
+      while( e == hipSuccess && launched < nchunks )
+      {
+         const std::atomic<int>& free = copied[(size_t)(launched - slots)];
+         if( free.load(std::memory_order_acquire) == 0 && launched >= upto )
+            return;
+         while( free.load(std::memory_order_acquire) == 0 )
+            std::this_thread::yield();
+         e = launch(launched++);
+      }
+   };
+   for( int64_t q = 0; q < nchunks && e == hipSuccess; ++q )
+   {
+      refill(q + 1);
+      if( e == hipSuccess )
+         e = hipEventSynchronize(c->ringev[q % slots]);
+      if( e != hipSuccess )
+         break;
+      ready.store(q + 1, std::memory_order_release);
+      if( th.empty() )
+         copyOut(q);
+      refill(0);
+   }
+   if( e != hipSuccess )
+      ready.store(nchunks + 1, std::memory_order_release);
+   else if( !th.empty() )
+      help();
+   for( auto& x : th )
+      x.join();
+   if( e != hipSuccess )
+      (void)hipStreamSynchronize(s);
+   HIPCHK(e);
+   return SAP_OKAY;
+}
+
+// ... into the caller's arrays
+static int downloadBounds(sap_context* c, const double2* src, int64_t nc, double* lb, double* ub)
+{
+   return downloadBounds(c, src, nc, [=](int64_t j0, int64_t n, const double* l, const double* u) {
+      memcpy(lb + j0, l, sizeof(double) * (size_t)n);
+      memcpy(ub + j0, u, sizeof(double) * (size_t)n);
+   });
+}
+
+extern "C" {
+
 int sap_bounds_upload(sap_bounds* b, int32_t v, const double* lb, const double* ub)
 {
    if( b == NULL || lb == NULL || ub == NULL || v >= b->nvec )
       return SAP_INVALIDDATA;
-   sap_matrix* m = b->mat;
-   hipStream_t s = m->ctx->stream;
-   HIPCHK(hipSetDevice(m->ctx->device));
-   const int64_t nc = m->ncols;
-   for( int64_t j = 0; j < nc; ++j )
-      if( lb[j] != lb[j] || ub[j] != ub[j] )
-         return SAP_INVALIDDATA;
-   HIPCHK(hipMemcpyAsync(b->stage, lb, sizeof(double) * (size_t)nc, hipMemcpyHostToDevice, s));
-   HIPCHK(hipMemcpyAsync(b->stage + nc, ub, sizeof(double) * (size_t)nc, hipMemcpyHostToDevice, s));
-   int32_t v0 = v < 0 ? 0 : v, v1 = v < 0 ? b->nvec : v + 1;
-   for( int32_t q = v0; q < v1; ++q )
-      k_interleave<<<gridFor((size_t)nc), SAP_BLOCK, 0, s>>>(b->V.bnd + (size_t)q * (size_t)nc, b->stage,
-         b->stage + nc, nc);
-   HIPCHK(hipGetLastError());
-   touchedVectors(b, v);
-   HIPCHK(hipStreamSynchronize(s));
+   HIPCHK(hipSetDevice(b->mat->ctx->device));
+   RCCHK(uploadBounds(b, v, lb, ub));
+   HIPCHK(hipStreamSynchronize(b->mat->ctx->stream));
+   b->mat->ctx->ringbusy = 0;
    return SAP_OKAY;
 }
 
@@ -5088,16 +5328,8 @@ int sap_bounds_download(sap_bounds* b, int32_t v, double* lb, double* ub)
    if( b == NULL || lb == NULL || ub == NULL || v < 0 || v >= b->nvec )
       return SAP_INVALIDDATA;
    sap_matrix* m = b->mat;
-   hipStream_t s = m->ctx->stream;
    HIPCHK(hipSetDevice(m->ctx->device));
-   const int64_t nc = m->ncols;
-   k_deinterleave<<<gridFor((size_t)nc), SAP_BLOCK, 0, s>>>(b->V.bnd + (size_t)v * (size_t)nc, b->stage,
-      b->stage + nc, nc);
-   HIPCHK(hipGetLastError());
-   HIPCHK(hipMemcpyAsync(lb, b->stage, sizeof(double) * (size_t)nc, hipMemcpyDeviceToHost, s));
-   HIPCHK(hipMemcpyAsync(ub, b->stage + nc, sizeof(double) * (size_t)nc, hipMemcpyDeviceToHost, s));
-   HIPCHK(hipStreamSynchronize(s));
-   return SAP_OKAY;
+   return downloadBounds(m->ctx, b->V.bnd + (size_t)v * (size_t)m->ncols, m->ncols, lb, ub);
 }
 
 int sap_bounds_copy(sap_bounds* dst, int32_t dv, const sap_bounds* src, int32_t sv)
@@ -5380,10 +5612,31 @@ struct ListSpec
    double2* bnd;      // cap (lb, ub)
 };
 
+// outcome of a call on vector 0 brought back by its last wait (k_land): device pointers into
+// the context's staging
+struct LandSpec
+{
+   double* lb;
+   double* ub;
+   uint32_t* hist;
+   uint32_t histmax;
+};
+
+static int enqueueLand(sap_bounds* b, const Params& P, const LandSpec* land)
+{
+   if( land == NULL )
+      return SAP_OKAY;
+   k_land<<<gridFor((size_t)b->mat->ncols), SAP_BLOCK, 0, b->mat->ctx->stream>>>(b->V, b->mat->ncols, P.maxrounds,
+      land->lb, land->ub, land->hist, land->histmax);
+   HIPCHK(hipGetLastError());
+   return SAP_OKAY;
+}
+
 // metan > 0: the outcomes of vectors 0..metan-1 (k_pack_meta) are also in b's landing area,
 // whose room the caller has made, when it returns, read by the call's last wait; with ls also
 // their change lists
-static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t metan = 0, const ListSpec* ls = NULL)
+static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t metan = 0, const ListSpec* ls = NULL,
+   const LandSpec* land = NULL)
 {
    RCCHK(ensureRanged(b, P));
    if( (P.flags & SAP_FLAG_HOSTLOOP) || b->graphbroken || !ensureGraphs(b, P) )
@@ -5395,6 +5648,11 @@ static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t m
          k_pack_meta<<<gridFor((size_t)metan), SAP_BLOCK, 0, s>>>(b->V, metan, (int32_t*)b->hdnd);
          HIPCHK(hipGetLastError());
          HIPCHK(hipStreamSynchronize(s));
+      }
+      if( land != NULL )
+      {
+         RCCHK(enqueueLand(b, P, land));
+         HIPCHK(hipStreamSynchronize(b->mat->ctx->stream));
       }
       return SAP_OKAY;
    }
@@ -5438,6 +5696,7 @@ static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t m
       if( metan > 0 )
          k_pack_meta<<<gridFor((size_t)metan), SAP_BLOCK, 0, s>>>(b->V, metan, (int32_t*)b->hdnd);
       HIPCHK(hipGetLastError());
+      RCCHK(enqueueLand(b, P, land));
       // the end event of the call rides on every group's synchronisation, so that the last
       // one needs no further round trip
       HIPCHK(hipEventRecord(c->ev[1], s));
@@ -5540,11 +5799,8 @@ static int createSingle(sap_matrix* m)
    return SAP_OKAY;
 }
 
-int sap_propagate_resident(sap_bounds* b, const sap_params* params, sap_stats* stats)
+static int propagateFirst(sap_bounds* b, const sap_params* params, sap_stats* stats, const LandSpec* land)
 {
-   if( b == NULL )
-      return SAP_INVALIDDATA;
-   RCCHK(checkParams(params));
    sap_matrix* m = b->mat;
    sap_context* c = m->ctx;
    HIPCHK(hipSetDevice(c->device));
@@ -5558,13 +5814,21 @@ int sap_propagate_resident(sap_bounds* b, const sap_params* params, sap_stats* s
    if( rc == SAP_OKAY && !b->V.dense )
       rc = queueAllRows(b, 1);
    if( rc == SAP_OKAY )
-      rc = runRounds(b, P, stats);
+      rc = runRounds(b, P, stats, 0, NULL, land);
    saved.restore(b->V);
    touchedVectors(b, 0);
    RCCHK(rc);
    if( stats )
       stats->result = c->hstatus->cutoff ? SAP_CUTOFF : (c->hstatus->nchg > 0 ? SAP_REDUCEDDOM : SAP_DIDNOTFIND);
    return SAP_OKAY;
+}
+
+int sap_propagate_resident(sap_bounds* b, const sap_params* params, sap_stats* stats)
+{
+   if( b == NULL )
+      return SAP_INVALIDDATA;
+   RCCHK(checkParams(params));
+   return propagateFirst(b, params, stats, NULL);
 }
 
 // destroy the round graphs of b; the stream they are launched on is drained first, so no
@@ -5615,6 +5879,8 @@ static bool histLess(const HistRec& a, const HistRec& b)
    return a.round != b.round ? a.round < b.round : a.colside < b.colside;
 }
 
+#define SAP_LAND_HIST 1024   // history entries that come back with the bounds of a small call
+
 int sap_propagate_reasons(sap_matrix* m, const sap_params* params, double* lb, double* ub, int64_t histcap,
    int64_t* nhist, int32_t* hround, int32_t* hcol, int32_t* hbound, double* hval, int32_t* hrow, int32_t* hrule,
    sap_conflict* conflict, sap_stats* stats)
@@ -5631,18 +5897,31 @@ int sap_propagate_reasons(sap_matrix* m, const sap_params* params, double* lb, d
    sap_bounds* b = m->rsingle;
    const Params P = toParams(params);
    const int64_t nc = m->ncols;
-   std::vector<double> lb0(lb, lb + nc), ub0(ub, ub + nc);
+   // up to SAP_RING_COLS columns the bounds and the first entries of the history come back with
+   // the call's last wait (the caller's arrays hold the start bounds until then)
+   const size_t nb = 8 * (size_t)nc;
+   const bool small = nc <= SAP_RING_COLS;
+   LandSpec land;
+   memset(&land, 0, sizeof(land));
    sap_stats local;
    for( int attempt = 0;; ++attempt )
    {
-      RCCHK(sap_bounds_upload(b, 0, lb0.data(), ub0.data()));
+      RCCHK(uploadBounds(b, 0, lb, ub, 2 * nb + SAP_LAND_HIST * sizeof(HistRec)));
+      if( small )
+      {
+         land.lb = (double*)(c->ringd + 2 * nb);
+         land.ub = (double*)(c->ringd + 3 * nb);
+         land.hist = (uint32_t*)(c->ringd + 4 * nb);
+         land.histmax = std::min<uint32_t>(SAP_LAND_HIST, b->V.histcap);
+      }
       k_reason_reset<<<gridFor((size_t)nc), SAP_BLOCK, 0, s>>>(b->V, nc);
       HIPCHK(hipGetLastError());
       memset(&local, 0, sizeof(local));
       b->V.nvec = 1;
       b->V.single = 1;
       RCCHK(beginCall(b, 1, 1));
-      RCCHK(runRounds(b, P, &local));
+      RCCHK(runRounds(b, P, &local, 0, NULL, small ? &land : NULL));
+      c->ringbusy = 0;
       const Status* h = c->hstatus;
       if( h->clogovf )
          return SAP_ERROR;   // cannot happen: the log holds two candidates per nonzero
@@ -5690,15 +5969,26 @@ int sap_propagate_reasons(sap_matrix* m, const sap_params* params, double* lb, d
          conflict->rules = ((f & RF_LB) ? (rr[0] & 1) : 0) | ((f & RF_UB) ? (rr[1] & 1) << 1 : 0);
       }
    }
-   if( !cut )
-      RCCHK(sap_bounds_download(b, 0, lb, ub));
+   std::vector<HistRec> hh((size_t)nh);
+   const bool landed = small && nh <= (int64_t)land.histmax;
+   if( landed && nh > 0 )
+      memcpy(hh.data(), c->ring + 4 * nb, sizeof(HistRec) * (size_t)nh);
+   if( !cut && small && nb > 0 )
+   {
+      memcpy(lb, c->ring + 2 * nb, nb);
+      memcpy(ub, c->ring + 3 * nb, nb);
+   }
+   else if( !cut )
+      RCCHK(downloadBounds(c, b->V.bnd, nc, lb, ub));
    if( nh > histcap )
       return SAP_NOMEMORY;
    if( nh > 0 )
    {
-      std::vector<HistRec> hh((size_t)nh);
-      HIPCHK(hipMemcpyAsync(hh.data(), b->V.hist, sizeof(HistRec) * (size_t)nh, hipMemcpyDeviceToHost, s));
-      HIPCHK(hipStreamSynchronize(s));
+      if( !landed )
+      {
+         HIPCHK(hipMemcpyAsync(hh.data(), b->V.hist, sizeof(HistRec) * (size_t)nh, hipMemcpyDeviceToHost, s));
+         HIPCHK(hipStreamSynchronize(s));
+      }
       std::sort(hh.begin(), hh.end(), histLess);
       for( int64_t q = 0; q < nh; ++q )
       {
@@ -5720,14 +6010,35 @@ int sap_propagate(sap_matrix* m, const sap_params* params, double* lb, double* u
    if( m == NULL || lb == NULL || ub == NULL )
       return SAP_INVALIDDATA;
    RCCHK(checkParams(params));
+   HIPCHK(hipSetDevice(m->ctx->device));
    if( m->single == NULL )
       RCCHK(createSingle(m));
-   RCCHK(sap_bounds_upload(m->single, 0, lb, ub));
+   sap_context* c = m->ctx;
+   sap_bounds* b = m->single;
+   const size_t nb = 8 * (size_t)m->ncols;
+   const bool small = m->ncols <= SAP_RING_COLS;
+   RCCHK(uploadBounds(b, 0, lb, ub, 2 * nb));
    sap_stats local;
    memset(&local, 0, sizeof(local));
-   RCCHK(sap_propagate_resident(m->single, params, &local));
-   if( local.result != SAP_CUTOFF )
-      RCCHK(sap_bounds_download(m->single, 0, lb, ub));
+   LandSpec land;
+   memset(&land, 0, sizeof(land));
+   if( small )
+   {
+      land.lb = (double*)(c->ringd + 2 * nb);
+      land.ub = (double*)(c->ringd + 3 * nb);
+   }
+   RCCHK(propagateFirst(b, params, &local, small ? &land : NULL));
+   c->ringbusy = 0;
+   if( local.result != SAP_CUTOFF && small )
+   {
+      if( nb > 0 )
+      {
+         memcpy(lb, c->ring + 2 * nb, nb);
+         memcpy(ub, c->ring + 3 * nb, nb);
+      }
+   }
+   else if( local.result != SAP_CUTOFF )
+      RCCHK(downloadBounds(c, b->V.bnd, m->ncols, lb, ub));
    if( stats )
       *stats = local;
    return SAP_OKAY;
@@ -6767,26 +7078,50 @@ int sap_propagate_packed(sap_matrix* m, const sap_params* params, double* lb, do
    sap_bounds* b = m->single;
    hipStream_t s = m->ctx->stream;
    const int32_t ns = m->nseg;
-   std::vector<double> in_lb(lb, lb + m->ncols), in_ub(ub, ub + m->ncols);
-   RCCHK(sap_bounds_upload(b, 0, lb, ub));
+   RCCHK(uploadBounds(b, 0, lb, ub));
    sap_stats local;
    memset(&local, 0, sizeof(local));
-   RCCHK(sap_propagate_resident(b, params, &local));
+   RCCHK(propagateFirst(b, params, &local, NULL));
+   m->ctx->ringbusy = 0;
+   // per-instance cutoffs and last rounds, and the call's first round, in one wait
    std::vector<int32_t> cut((size_t)ns), vr((size_t)ns);
+   char* h = NULL;
+   const size_t ub4 = sizeof(int32_t) * (size_t)ns;
+   RCCHK(downloadArea(b, 2 * ub4 + sizeof(int32_t), &h));
+   RCCHK(download(b, h, b->V.vcutoff, ub4));
+   RCCHK(download(b, h + ub4, b->V.vrounds, ub4));
+   RCCHK(download(b, h + 2 * ub4, b->V.vstart, sizeof(int32_t)));
+   // an instance has changed bounds when some arriving value differs from the caller's
+   std::vector<std::atomic<int>> changed((size_t)ns);
+   for( auto& x : changed )
+      x = 0;
+   RCCHK(downloadBounds(m->ctx, b->V.bnd, m->ncols, [&](int64_t j0, int64_t n, const double* l, const double* u) {
+      int32_t q = 0;
+      if( ns > 1 )
+         q = (int32_t)(std::upper_bound(m->coloff->begin(), m->coloff->end(), j0) - m->coloff->begin()) - 1;
+      for( int64_t j = j0; j < j0 + n; ++q )
+      {
+         const int64_t e = std::min(j0 + n, ns > 1 ? (*m->coloff)[(size_t)q + 1] : m->ncols);
+         int diff = 0;
+         for( int64_t k = j; k < e; ++k )
+            diff |= (lb[k] != l[k - j0]) | (ub[k] != u[k - j0]);
+         if( diff )
+            changed[(size_t)q] = 1;
+         j = e;
+      }
+      memcpy(lb + j0, l, sizeof(double) * (size_t)n);
+      memcpy(ub + j0, u, sizeof(double) * (size_t)n);
+   }));
+   if( m->ncols == 0 )
+      HIPCHK(hipStreamSynchronize(s));
    int32_t vs = 0;
-   HIPCHK(hipMemcpyAsync(cut.data(), b->V.vcutoff, sizeof(int32_t) * (size_t)ns, hipMemcpyDeviceToHost, s));
-   HIPCHK(hipMemcpyAsync(vr.data(), b->V.vrounds, sizeof(int32_t) * (size_t)ns, hipMemcpyDeviceToHost, s));
-   HIPCHK(hipMemcpyAsync(&vs, b->V.vstart, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-   HIPCHK(hipStreamSynchronize(s));
-   RCCHK(sap_bounds_download(b, 0, lb, ub));
+   memcpy(cut.data(), h, ub4);
+   memcpy(vr.data(), h + ub4, ub4);
+   memcpy(&vs, h + 2 * ub4, sizeof(int32_t));
    int32_t anycut = 0;
    for( int32_t q = 0; q < ns; ++q )
    {
-      const int64_t c0 = ns > 1 ? (*m->coloff)[(size_t)q] : 0, c1 = ns > 1 ? (*m->coloff)[(size_t)q + 1] : m->ncols;
-      bool changed = false;
-      for( int64_t j = c0; j < c1 && !changed; ++j )
-         changed = lb[j] != in_lb[(size_t)j] || ub[j] != in_ub[(size_t)j];
-      const int32_t r = cut[(size_t)q] ? SAP_CUTOFF : (changed ? SAP_REDUCEDDOM : SAP_DIDNOTFIND);
+      const int32_t r = cut[(size_t)q] ? SAP_CUTOFF : (changed[(size_t)q] ? SAP_REDUCEDDOM : SAP_DIDNOTFIND);
       anycut |= cut[(size_t)q];
       if( result )
          result[q] = r;

@@ -1,0 +1,71 @@
+"""Host bound arrays to the device and back at the sizes where their route changes: one chunk of
+32,768 columns (staged in one piece, read back with the call's own wait), two and more chunks
+(copied out by helper threads), more chunks than there are slots.  Every value comes back as it
+was, a NaN anywhere is refused and changes nothing, and the calls on host arrays agree with the
+oracle's Jacobi twin."""
+import numpy as np
+import pytest
+
+import scip_amd as sa
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 32_767, 32_768, 32_769, 65_537, 98_304, 262_144, 262_145, 300_001]
+
+
+@pytest.mark.parametrize("ncols", SIZES)
+def test_round_trip(gpu_ctx, ncols):
+    print(f"[case] transfer ncols={ncols}", flush=True)
+    rng = np.random.default_rng(ncols)
+    inst = sa.Instance(rowptr=np.array([0, 1], np.int64), colidx=np.array([ncols - 1], np.int32), vals=np.ones(1),
+                       lhs=np.array([-1e20]), rhs=np.array([1e20]), integral=np.zeros(ncols, np.uint8),
+                       lb=-rng.random(ncols), ub=rng.random(ncols))
+    inst.lb[0] = -1e20
+    mat = sa.Matrix(gpu_ctx, inst)
+    b = sa.Bounds(mat, 2)
+    b.upload(inst.lb, inst.ub)
+    b.upload(inst.lb - 1.0, inst.ub + 1.0, v=1)   # the staging of the first upload is free again
+    for v, off in ((0, 0.0), (1, 1.0)):
+        lb, ub = b.download(v)
+        assert np.array_equal(lb, inst.lb - off) and np.array_equal(ub, inst.ub + off), v
+    for at in {0, ncols // 2, ncols - 1}:
+        for side in (0, 1):
+            bad = [inst.lb + 5.0, inst.ub + 5.0]
+            bad[side][at] = np.nan
+            with pytest.raises(sa.SapError) as e:
+                b.upload(*bad, v=0)
+            assert e.value.rc == sa.SAP_INVALIDDATA
+            with pytest.raises(sa.SapError):
+                mat.propagate(*bad)
+    lb, ub = b.download(0)
+    assert np.array_equal(lb, inst.lb) and np.array_equal(ub, inst.ub)
+    b.close()
+    mat.close()
+
+
+@pytest.mark.parametrize("ncols", [32_768, 32_769, 262_145])
+def test_calls(gpu_ctx, ncols):
+    print(f"[case] calls ncols={ncols}", flush=True)
+    inst = sa.gen_mixed(ncols // 4, ncols, seed=ncols % 97, planted=True)
+    ol, ou, orr = orc.propagate_jacobi(orc.OMatrix.from_instance(inst), inst.lb, inst.ub)
+    assert not orr["cutoff"] and orr["nchgbds"] > 1024   # more than the history entries that come with the bounds
+    mat = sa.Matrix(gpu_ctx, inst)
+    for flags in (0, sa.SAP_FLAG_HOSTLOOP):
+        lb, ub, st = mat.propagate(params=sa.default_params(flags=flags))
+        assert np.array_equal(lb, ol) and np.array_equal(ub, ou) and st["rounds"] == orr["rounds"]
+    r = mat.propagate_reasons()
+    assert np.array_equal(r["lb"], ol) and np.array_equal(r["ub"], ou) and r["nhist"] == orr["nchgbds"]
+    r = mat.propagate_reasons(ol, ou)   # nothing left to do: an empty history
+    assert np.array_equal(r["lb"], ol) and np.array_equal(r["ub"], ou) and r["nhist"] == 0
+    mat.close()
+    # packed: instance 0 changes, instance 1 is at its fixpoint, instance 2 has no rows
+    done = sa.Instance(**{**inst.__dict__, "lb": ol, "ub": ou})
+    none = sa.Instance(rowptr=np.zeros(1, np.int64), colidx=np.zeros(0, np.int32), vals=np.zeros(0), lhs=np.zeros(0),
+                       rhs=np.zeros(0), integral=np.zeros(7, np.uint8), lb=np.zeros(7), ub=np.ones(7))
+    packed = sa.PackedMatrix(gpu_ctx, [inst, done, none])
+    lb, ub, res, rnd, _ = packed.propagate_packed()
+    assert res.tolist() == [sa.SAP_REDUCEDDOM, sa.SAP_DIDNOTFIND, sa.SAP_DIDNOTFIND]
+    assert rnd[0] == orr["rounds"]
+    assert np.array_equal(lb, np.concatenate([ol, ol, none.lb])) and np.array_equal(ub, np.concatenate([ou, ou, none.ub]))
+    packed.close()
