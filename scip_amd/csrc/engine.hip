@@ -24,7 +24,7 @@
 // Bins: in the dense mode rows of up to 128 nonzeros are swept in tiles of 64 lanes holding
 // 1, 2 or 4 nonzeros each (rows packed first-fit decreasing); in the sparse mode rows of
 // length <= 4/8/16/32/64 are swept by groups of that many lanes; longer rows by one wavefront
-// (64-element chunks), the longest by a whole workgroup.  All tilings compute the same
+// (256-element chunks), the longest by a whole workgroup.  All tilings compute the same
 // canonical tree, so the result does not depend on the binning.
 #include <hip/hip_runtime.h>
 
@@ -235,6 +235,7 @@ struct HistRec
 struct Layout
 {
    int32_t blockstart[SAP_NKINDS + 1];
+   int32_t longfirst;   // the workgroups start in reverse order: the longest rows' before the tiles'
 };
 
 #define KEY_NEG_INF ((long long)0x800FFFFFFFFFFFFFLL)   // dkey(-inf)
@@ -1837,10 +1838,16 @@ __device__ __forceinline__ void sweepTilesW(const Mat& M, const Vec& V, const Pa
 }
 
 // ------------------------------------------------------------------------------------------
-// sweep of one long row by one wavefront: the chunks [c0, c0+nch) of 64 positions form an
-// aligned subtree of the canonical tree; the wave returns its root (all lanes) and the
-// per-lane counters / maxactdelta contributions.
+// sweep of one long row by one wavefront: the chunks [c0, c0+nch) of SAP_CHUNK positions, four
+// consecutive ones per lane, form an aligned subtree of the canonical tree; the wave returns
+// its root, the infinity / huge counts and the maxactdelta (all lanes).  A long row is a chain
+// of loads, gathers and shuffles that nothing else in its wavefront hides: with one position
+// per lane (chunks of 64) it had four times the gather waits, and six tree levels per 64
+// positions instead of per 256.
 // ------------------------------------------------------------------------------------------
+#define SAP_CHUNKW 4
+#define SAP_CHUNK (SAP_CHUNKW * SAP_WAVE)
+
 struct WavePart
 {
    DD minact;
@@ -1850,39 +1857,75 @@ struct WavePart
    int inf;
 };
 
-__device__ __forceinline__ WavePart waveSubtree(const Mat& M, const Params& P, const double2* bnd, int64_t s, int64_t n, int64_t c0,
-   int64_t nch, bool allbin)
+// the nonzeros at positions SAP_CHUNK * c + SAP_CHUNKW * lane + i of a row (those past its end: none)
+__device__ __forceinline__ void loadChunk(const Mat& M, const double2* bnd, int64_t s, int64_t n, int64_t c,
+   Elem (&e)[SAP_CHUNKW])
+{
+   const int64_t p0 = c * SAP_CHUNK + SAP_CHUNKW * ((int)threadIdx.x & (SAP_WAVE - 1));
+#pragma unroll
+   for( int i = 0; i < SAP_CHUNKW; ++i )
+   {
+      e[i].a = 1.0;
+      e[i].lb = 0.0;
+      e[i].ub = 0.0;
+      e[i].j = 0;
+      e[i].cf = 0;
+      if( p0 + i < n )
+         e[i] = loadElem(M, bnd, s + p0 + i);
+   }
+}
+
+__device__ __forceinline__ WavePart waveSubtree(const Mat& M, const Params& P, const double2* bnd, int64_t s, int64_t n,
+   int64_t c0, int64_t nch, bool allbin)
 {
    const int lane = (int)threadIdx.x & (SAP_WAVE - 1);
    WavePart w;
    DD stmin = { 0.0, 0.0 }, stmax = { 0.0, 0.0 };   // level `lane` of the binary-counter stack
-   int32_t k0 = 0, k1 = 0, k2 = 0, k3 = 0, k4 = 0, k5 = 0, k6 = 0, k7 = 0;
+#pragma unroll
+   for( int q = 0; q < 8; ++q )
+      w.c[q] = 0;
    double mad = 0.0;
-   int inf = 0;
+   bool inf = false;
    int64_t cnt = 0;
    for( int64_t c = c0; c < c0 + nch; ++c )
    {
-      const int64_t pos = c * SAP_WAVE + lane;
-      double cmin = 0.0, cmax = 0.0;
-      if( pos < n )
+      const int64_t p0 = c * SAP_CHUNK + SAP_CHUNKW * lane;
+      Elem e[SAP_CHUNKW];
+      loadChunk(M, bnd, s, n, c, e);
+      DD vmin[SAP_CHUNKW], vmax[SAP_CHUNKW];
+#pragma unroll
+      for( int i = 0; i < SAP_CHUNKW; ++i )
       {
-         Elem e = loadElem(M, bnd, s + pos);
-         int kmin, kmax;
-         double md;
-         bool mi;
-         elemContrib(P, e, allbin, cmin, cmax, kmin, kmax, md, mi);
-         k0 += (kmin == 1);
-         k1 += (kmin == 2);
-         k2 += (kmin == 3);
-         k3 += (kmin == 4);
-         k4 += (kmax == 1);
-         k5 += (kmax == 2);
-         k6 += (kmax == 3);
-         k7 += (kmax == 4);
-         mad = dmax(mad, md);
-         inf |= mi ? 1 : 0;
+         double cmin = 0.0, cmax = 0.0;
+         int kmin = 0, kmax = 0;
+         if( p0 + i < n )
+         {
+            double md;
+            bool mi;
+            elemContrib(P, e[i], allbin, cmin, cmax, kmin, kmax, md, mi);
+            mad = dmax(mad, md);
+            inf = inf || mi;
+         }
+         if( __ballot((kmin | kmax) != 0) != 0 )
+#pragma unroll
+            for( int q = 0; q < 4; ++q )
+            {
+               w.c[q] += __popcll(__ballot(kmin == q + 1));
+               w.c[4 + q] += __popcll(__ballot(kmax == q + 1));
+            }
+         vmin[i] = { cmin, 0.0 };
+         vmax[i] = { cmax, 0.0 };
       }
-      DD rmin = { cmin, 0.0 }, rmax = { cmax, 0.0 };
+      // the levels inside the lane, then those across the wavefront
+#pragma unroll
+      for( int h = 1; h < SAP_CHUNKW; h <<= 1 )
+#pragma unroll
+         for( int i = 0; i < SAP_CHUNKW; i += 2 * h )
+         {
+            vmin[i] = pairAdd(vmin[i], vmin[i + h]);
+            vmax[i] = pairAdd(vmax[i], vmax[i + h]);
+         }
+      DD rmin = vmin[0], rmax = vmax[0];
 #pragma unroll
       for( int off = 1; off < SAP_WAVE; off <<= 1 )
       {
@@ -1929,56 +1972,44 @@ __device__ __forceinline__ WavePart waveSubtree(const Mat& M, const Params& P, c
    }
    w.minact = amin;
    w.maxact = amax;
-   // counters and maxactdelta reduced over the wave (pairs of 32-bit counters per 64-bit lane word)
-   long long p01 = ((long long)k1 << 32) | (unsigned)k0, p23 = ((long long)k3 << 32) | (unsigned)k2;
-   long long p45 = ((long long)k5 << 32) | (unsigned)k4, p67 = ((long long)k7 << 32) | (unsigned)k6;
 #pragma unroll
    for( int off = 1; off < SAP_WAVE; off <<= 1 )
-   {
-      p01 += __shfl_xor(p01, off, SAP_WAVE);
-      p23 += __shfl_xor(p23, off, SAP_WAVE);
-      p45 += __shfl_xor(p45, off, SAP_WAVE);
-      p67 += __shfl_xor(p67, off, SAP_WAVE);
-   }
-   w.c[0] = (int32_t)(p01 & 0xFFFFFFFF);
-   w.c[1] = (int32_t)(p01 >> 32);
-   w.c[2] = (int32_t)(p23 & 0xFFFFFFFF);
-   w.c[3] = (int32_t)(p23 >> 32);
-   w.c[4] = (int32_t)(p45 & 0xFFFFFFFF);
-   w.c[5] = (int32_t)(p45 >> 32);
-   w.c[6] = (int32_t)(p67 & 0xFFFFFFFF);
-   w.c[7] = (int32_t)(p67 >> 32);
-#pragma unroll
-   for( int off = 1; off < SAP_WAVE; off <<= 1 )
-   {
       mad = dmax(mad, shflXorD(mad, off));
-      inf |= __shfl_xor(inf, off, SAP_WAVE);
-   }
    w.mad = mad;
-   w.inf = inf;
+   w.inf = __ballot(inf) != 0 ? 1 : 0;
    return w;
 }
 
+// the nonzero of one lane, none past the end of its row
+__device__ __forceinline__ Elem loadOr(const Mat& M, const double2* bnd, int64_t k, bool has)
+{
+   Elem e;
+   e.a = 1.0;
+   e.lb = 0.0;
+   e.ub = 0.0;
+   e.j = 0;
+   e.cf = 0;
+   if( has )
+      e = loadElem(M, bnd, k);
+   return e;
+}
+
+// candidates of the chunks [c0, c0+nch), a wavefront's width of positions at a time (four per lane
+// at once, held across the drain, spill 200 registers; loading the next ones ahead gains nothing)
 template <bool R>
 __device__ __forceinline__ void candidatesRange(const Mat& M, const Vec& V, const Params& P, WaveQueue& Q,
    const RowState& rs, const RowDecision& d, double lhs, double rhs, const double2* bnd, int64_t s, int64_t n,
    int64_t c0, int64_t nch, int32_t row, int32_t v, int32_t round)
 {
    const int lane = (int)threadIdx.x & (SAP_WAVE - 1);
-   for( int64_t c = c0; c < c0 + nch; ++c )
+   int64_t p = c0 * SAP_CHUNK;
+   const int64_t end = (c0 + nch) * SAP_CHUNK < n ? (c0 + nch) * SAP_CHUNK : n;
+   for( ; p < end; p += SAP_WAVE )
    {
-      const int64_t pos = c * SAP_WAVE + lane;
-      const bool has = pos < n;
-      Elem e;
-      e.a = 1.0;
-      e.lb = 0.0;
-      e.ub = 0.0;
-      e.j = 0;
-      e.cf = 0;
-      if( has )
-         e = loadElem(M, bnd, s + pos);
+      const bool has = p + lane < end;
+      const Elem e = loadOr(M, bnd, s + p + lane, has);
       const bool pass = has && screenElem(P, rs, d, lhs, rhs, e);
-      pushQueue(M, V, P, Q, pass, s + pos, e, row, v, rs, d, round);
+      pushQueue(M, V, P, Q, pass, s + p + lane, e, row, v, rs, d, round);
       maybeDrain<R>(M, V, P, Q, round);
    }
 }
@@ -2006,7 +2037,7 @@ __device__ __forceinline__ void sweepWaves(const Mat& M, const Vec& V, const Par
       const double2* bnd = V.bnd + (size_t)v * (size_t)M.ncols;
       const int64_t s = M.rowptr[row];
       const int64_t n = M.rowptr[row + 1] - s;
-      const int64_t nch = (n + SAP_WAVE - 1) / SAP_WAVE;
+      const int64_t nch = (n + SAP_CHUNK - 1) / SAP_CHUNK;
       const double2 sides = M.sides[row];
       const bool allbin = (M.rowflags[row] & 1) != 0;
       WavePart w = waveSubtree(M, P, bnd, s, n, 0, nch, allbin);
@@ -2061,7 +2092,7 @@ __device__ __forceinline__ void sweepBlocks(const Mat& M, const Vec& V, const Pa
       const double2* bnd = V.bnd + (size_t)v * (size_t)M.ncols;
       const int64_t s = M.rowptr[row];
       const int64_t n = M.rowptr[row + 1] - s;
-      const int64_t nch = (n + SAP_WAVE - 1) / SAP_WAVE;
+      const int64_t nch = (n + SAP_CHUNK - 1) / SAP_CHUNK;
       int64_t P2 = 1;
       while( P2 < nch )
          P2 <<= 1;
@@ -2199,13 +2230,13 @@ __global__ __launch_bounds__(SAP_BLOCK, 4) void k_sweep(Mat M, Vec V, Params P, 
    int kind = 0, lblock, nblocks;
    if( D && W.dense )
    {
-      const int blk = (int)blockIdx.x;
+      const int blk = L.longfirst ? L.blockstart[SAP_NKINDS] - 1 - (int)blockIdx.x : (int)blockIdx.x;
+      if( blk < 0 || blk >= L.blockstart[SAP_NKINDS] )
+         return;   // a workgroup that only listed rounds use
       while( kind < SAP_NKINDS - 1 && blk >= L.blockstart[kind + 1] )
          ++kind;
       lblock = blk - L.blockstart[kind];
       nblocks = L.blockstart[kind + 1] - L.blockstart[kind];
-      if( lblock >= nblocks )
-         return;   // a workgroup that only listed rounds use
    }
    else if( !listShare(M, *st, I.round & 1, kind, lblock, nblocks) )
       return;
@@ -3723,7 +3754,7 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_row_activities(Mat M, Params P, c
    {
       const int64_t s = M.rowptr[row];
       const int64_t n = M.rowptr[row + 1] - s;
-      const int64_t nch = (n + SAP_WAVE - 1) / SAP_WAVE;
+      const int64_t nch = (n + SAP_CHUNK - 1) / SAP_CHUNK;
       WavePart w = waveSubtree(M, P, bnd, s, n, 0, nch, (M.rowflags[row] & 1) != 0);
       if( lane == 0 )
       {
@@ -5357,10 +5388,11 @@ static Layout makeLayout(const sap_bounds* b)
       SAP_BLOCK / 16, SAP_BLOCK / 32, SAP_BLOCK / 64, SAP_BLOCK / SAP_WAVE, SAP_BLOCK / SAP_WAVE, 1 };
    static const int kCap[SAP_NKINDS] = { 4096, 2048, 2048, 2048, 2048, 2048, 2048, 2048, 2048, 1024 };
    const int tb = m->tuning.tilebins, rb = m->tuning.rowbins;
-   int acc = 0;
+   size_t blocks[SAP_NKINDS], units[SAP_NKINDS], all = 0, sum = 0;
+   // rough time of an item against a tile's 4, per wavefront (a row of kind 9 takes four)
+   static const int kUnits[SAP_NKINDS] = { 4, 4, 4, 4, 4, 4, 4, 3, 5, 64 };
    for( int q = 0; q < SAP_NKINDS; ++q )
    {
-      L.blockstart[q] = acc;
       const int bin = q - 1;
       size_t items;
       if( q == 0 )
@@ -5370,14 +5402,45 @@ static Layout makeLayout(const sap_bounds* b)
       else
          items = nvec * (size_t)(m->binstart[q] - m->binstart[q - 1]);
       const int per = (bin >= 1 && bin <= rb) ? SAP_BLOCK : kPerBlock[q];   // one row per lane
-      size_t blocks = (items + per - 1) / per;
+      blocks[q] = (items + per - 1) / per;
       const size_t cap = std::max<size_t>(64, (size_t)kCap[q] * (size_t)m->tuning.capscale / 100);
-      if( blocks > cap )
-         blocks = cap;
-      // the tiles' grid-stride loop runs in generations of resident workgroups: at most one
-      if( q == 0 && m->ctx->resident > 0 && blocks > (size_t)m->ctx->resident )
-         blocks = (size_t)m->ctx->resident;
-      acc += (int)blocks;
+      blocks[q] = std::min(blocks[q], cap);
+      units[q] = q >= 1 && q <= 6 ? 0 : items * (size_t)kUnits[q];
+      all += units[q];
+      sum += blocks[q];
+   }
+   // The tiles' grid-stride loop runs in one generation of resident workgroups.  When they alone
+   // fill the device, the wavefronts of the long rows start as the first tiles end, and their
+   // chain of 12-14 us is the tail of every scanned round.  With few tiles per wavefront the
+   // long rows therefore start first, in a share of the places that follows their work, and the
+   // tiles take the rest: the four scanned sweeps of 100k rows (1.3 tiles per wavefront) 52 / 49
+   // / 45 / 41 -> 46 / 42 / 38 / 32 us, the first four of 300k rows (3.8) 94 / 98 / 93 / 79 -> 99 /
+   // 91 / 84 / 68 us.  With many (1M rows, 12.7) the places cost the tiles more than the tail:
+   // 280 -> 288 us.
+   const size_t res = (size_t)std::max(m->ctx->resident, 0);
+   L.longfirst = 0;
+   if( b->V.dense && res > 0 && blocks[0] > 0 )
+   {
+      size_t room = res;
+      if( sum > res && units[0] / (size_t)kUnits[0] <= 8 * res * (SAP_BLOCK / SAP_WAVE) )
+      {
+         size_t others = 0;
+         for( int q = 1; q < SAP_NKINDS; ++q )
+         {
+            if( units[q] > 0 )
+               blocks[q] = std::min(blocks[q], std::max<size_t>(1, (res * units[q] + all - 1) / all));
+            others += blocks[q];
+         }
+         room = std::max(res / 2, others < res ? res - others : 0);
+         L.longfirst = 1;
+      }
+      blocks[0] = std::min(blocks[0], room);
+   }
+   int acc = 0;
+   for( int q = 0; q < SAP_NKINDS; ++q )
+   {
+      L.blockstart[q] = acc;
+      acc += (int)blocks[q];
    }
    L.blockstart[SAP_NKINDS] = acc;
    return L;
