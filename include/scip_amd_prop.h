@@ -349,8 +349,8 @@ int sap_slots_collect(sap_bounds* bnd, int32_t n, const int32_t* slots, int32_t*
  * ncols doubles, the node's bounds, overwritten with the fixpoint unless the result is a
  * cutoff.  The work arrays live in one static device array per GPU (about 66 MiB, held until
  * the process ends), so the matrix may have at most 2^20 columns and 2^20 rows and one
- * instance, and ranged-row propagation is refused (SAP_INVALIDDATA); rounds run from a host
- * loop.  Calls on one GPU share that array: calls that overlap on one GPU (several threads or
+ * instance, and ranged-row propagation is refused (SAP_INVALIDDATA); rounds are enqueued launch
+ * by launch.  Calls on one GPU share that array: calls that overlap on one GPU (several threads or
  * contexts) race.  The results equal sap_propagate's. */
 int sap_propagate_device_noalloc(sap_matrix* mat, const sap_params* params, double* dlb, double* dub,
    sap_stats* stats);

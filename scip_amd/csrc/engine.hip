@@ -3688,6 +3688,40 @@ __global__ void k_deinterleave(const double2* src, double* lb, double* ub, int64
    }
 }
 
+// no-allocation entry point: the static scratch keeps the last call's contents, so everything a
+// call reads before writing is cleared, and the bounds are taken over, in one launch (eleven
+// fills and an interleave took 2 us each and 5-10 us to enqueue)
+__global__ void k_noalloc_begin(Vec V, const double* lb, const double* ub, int64_t ncols, int64_t nrows)
+{
+   const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+   for( int64_t j = i0; j < ncols; j += step )
+   {
+      V.bnd[j] = make_double2(lb[j], ub[j]);
+      V.clb[j] = KEY_NEG_INF;
+      V.cub[j] = KEY_POS_INF;
+      if( V.hasforced )
+      {
+         V.flb[j] = KEY_NEG_INF;
+         V.fub[j] = KEY_POS_INF;
+      }
+      V.coltag[j] = 0;
+      V.chgtag[j] = 0;
+   }
+   for( int64_t r = i0; r < nrows; r += step )
+   {
+      V.rowmark[r] = 0;
+      V.redundant[r] = 0;
+   }
+   for( int64_t w = i0; w < (int64_t)(sizeof(Status) / 4); w += step )
+      ((int32_t*)V.st)[w] = 0;
+   if( i0 == 0 )
+   {
+      V.vpend[0] = 0;
+      V.vstart[0] = 0;
+      V.vlogn[0] = 0;
+   }
+}
+
 // the outcome of a call on vector 0, written to mapped host memory after every round group once
 // the call has ended (its done flag, or the stop test the host applies after the group): the
 // bounds (lb NULL: not asked for), and the first histmax entries of the reason history as 32-bit
@@ -3883,6 +3917,7 @@ struct sap_bounds
    Status* dstatus;
    int64_t device_bytes;
    double* stage;   // device staging for host lb/ub (2*ncols)
+   int2* wlmem;     // the worklists and the touched list (V.wl, V.touched)
    int32_t roundbase;
    int32_t graphbroken;   // capture failed once: use the host-driven loop
    int32_t redgen;        // generation of the redundant-row flags of the last call (0: none yet)
@@ -3931,6 +3966,7 @@ struct sap_bounds
    size_t hdncap;
    // vectors 0..logmax-1 may hold change-log bits that no collection has cleared yet
    int32_t logmax;
+   int32_t direct;  // round groups are enqueued launch by launch, not as captured graphs
    int32_t begun;   // the last beginCall also began the call's first round
    int32_t lastrounds;   // rounds of the last graph-driven call on b (predicts the next one's)
 };
@@ -4959,10 +4995,7 @@ static void boundsRelease(sap_bounds* b)
    for( int e = 0; e < 2; ++e )
       if( b->evs[e] != NULL )
          (void)hipEventDestroy(b->evs[e]);
-   for( int p = 0; p < 2; ++p )
-      for( int q = 0; q < SAP_NBINS; ++q )
-         (void)hipFree(V.wl[p][q]);
-   (void)hipFree(V.touched);
+   (void)hipFree(b->wlmem);
    (void)hipFree(b->dstatus);
    (void)hipFree(b->stage);
    for( int g = 0; g < SAP_NGRAPHS; ++g )
@@ -5072,10 +5105,26 @@ int sap_bounds_create_mode(sap_matrix* m, int32_t nvec, int32_t mode, sap_bounds
    BALLOC(b->outoff, (size_t)nvec + 1);
    BALLOC(b->ident, nvec);
    listLimits(m, V);
-   for( int p = 0; p < 2; ++p )
-      for( int q = 0; q < SAP_NBINS; ++q )
-         BALLOC(V.wl[p][q], std::min((size_t)nvec * (size_t)(m->binstart[q + 1] - m->binstart[q]), (size_t)V.listcap));
-   BALLOC(V.touched, std::min(NC, (size_t)V.touchcap));
+   {
+      // one allocation for the 18 row lists and the touched list (each 256-byte aligned)
+      size_t len[2 * SAP_NBINS + 1], total = 0;
+      for( int q = 0; q <= 2 * SAP_NBINS; ++q )
+      {
+         const size_t n = q < 2 * SAP_NBINS
+            ? std::min((size_t)nvec * (size_t)(m->binstart[q / 2 + 1] - m->binstart[q / 2]), (size_t)V.listcap)
+            : std::min(NC, (size_t)V.touchcap);
+         len[q] = (n + 31) & ~(size_t)31;
+         total += len[q];
+      }
+      BALLOC(b->wlmem, total);
+      int2* next = b->wlmem;
+      for( int q = 0; q < 2 * SAP_NBINS; ++q )
+      {
+         V.wl[q & 1][q / 2] = next;
+         next += len[q];
+      }
+      V.touched = next;
+   }
    BALLOC(b->dstatus, 1);
    BALLOC(b->stage, 2 * (size_t)m->ncols);
 #undef BALLOC
@@ -5702,7 +5751,7 @@ static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t m
    const LandSpec* land = NULL)
 {
    RCCHK(ensureRanged(b, P));
-   if( (P.flags & SAP_FLAG_HOSTLOOP) || b->graphbroken || !ensureGraphs(b, P) )
+   if( (P.flags & SAP_FLAG_HOSTLOOP) || b->graphbroken || (!b->direct && !ensureGraphs(b, P)) )
    {
       RCCHK(runRoundsHost(b, P, stats));
       if( metan > 0 )
@@ -5724,6 +5773,8 @@ static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t m
    double sweepms = 0.0;
    int64_t launches = 0;
    int32_t prev = 0;
+   const Mat M0 = toMat(b->mat);
+   const Layout L0 = makeLayout(b);
    HIPCHK(hipEventRecord(c->ev[0], s));
    for( int it = 0;; ++it )
    {
@@ -5740,17 +5791,18 @@ static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t m
       static const int kSchedule[3] = { 0, 2, 1 };   // 2, 4, 8 rounds
       if( it == 0 )
       {
-         const Mat M0 = toMat(b->mat);
-         const Layout L0 = makeLayout(b);
          enqueueRound(b, M0, P, L0, s, NULL, NULL, b->begun != 0);
          b->begun = 0;
          HIPCHK(hipGetLastError());
-         if( b->V.nvec > 1 || b->lastrounds > 1 )
+         if( !b->direct && (b->V.nvec > 1 || b->lastrounds > 1) )
          {
             HIPCHK(hipGraphLaunch(b->graph[kSchedule[0]].exec, s));
             it = 1;
          }
       }
+      else if( b->direct )
+         for( int r = 0; r < (it < 3 ? 2 << (it - 1) : SAP_GRAPH_LONG); ++r )
+            enqueueRound(b, M0, P, L0, s, NULL, NULL);
       else
          HIPCHK(hipGraphLaunch(b->graph[kSchedule[it < 3 ? it - 1 : 2]].exec, s));
       // the status goes to mapped host memory by a copy kernel on the stream
@@ -7417,7 +7469,7 @@ int sap_propagate_device_noalloc(sap_matrix* m, const sap_params* params, double
    memset(&b, 0, sizeof(b));
    b.mat = m;
    b.nvec = 1;
-   b.graphbroken = 1;   // rounds from the host loop: capturing a graph would allocate
+   b.direct = 1;   // capturing a graph would allocate
    b.internal = 1;
    Vec& V = b.V;
    V.nvec = 1;
@@ -7459,29 +7511,15 @@ int sap_propagate_device_noalloc(sap_matrix* m, const sap_params* params, double
    V.st = b.dstatus;
    if( (size_t)(next - c->scratch) > SAP_NOALLOC_BYTES )
       return SAP_ERROR;   // cannot happen: the size covers the largest admitted matrix
-   // the array keeps the last call's contents: everything a call reads before writing is
-   // cleared with fill kernels (no memset nodes, so a caller may capture the call)
-   k_fill_i64<<<gridFor(nc), SAP_BLOCK, 0, s>>>(V.clb, KEY_NEG_INF, nc);
-   k_fill_i64<<<gridFor(nc), SAP_BLOCK, 0, s>>>(V.cub, KEY_POS_INF, nc);
-   if( m->hasforced )
-   {
-      k_fill_i64<<<gridFor(nc), SAP_BLOCK, 0, s>>>(V.flb, KEY_NEG_INF, nc);
-      k_fill_i64<<<gridFor(nc), SAP_BLOCK, 0, s>>>(V.fub, KEY_POS_INF, nc);
-   }
-   k_fill_i32<<<gridFor(nc), SAP_BLOCK, 0, s>>>(V.coltag, 0, nc);
-   k_fill_i32<<<gridFor(nc), SAP_BLOCK, 0, s>>>(V.chgtag, 0, nc);
-   k_fill_i32<<<gridFor(nr), SAP_BLOCK, 0, s>>>(V.rowmark, 0, nr);
-   k_fill_i32<<<1, SAP_BLOCK, 0, s>>>(V.vpend, 0, 1);
-   k_fill_i32<<<1, SAP_BLOCK, 0, s>>>(V.vstart, 0, 1);
-   k_fill_i32<<<1, SAP_BLOCK, 0, s>>>(V.vlogn, 0, 1);
-   k_fill_i32<<<gridFor(sizeof(Status) / 4), SAP_BLOCK, 0, s>>>((int32_t*)b.dstatus, 0, sizeof(Status) / 4);
-   k_interleave<<<gridFor(nc), SAP_BLOCK, 0, s>>>(V.bnd, dlb, dub, (int64_t)nc);
+   k_noalloc_begin<<<gridFor(std::max(std::max(nc, nr), sizeof(Status) / 4)), SAP_BLOCK, 0, s>>>(V, dlb, dub,
+      (int64_t)nc, (int64_t)nr);
    HIPCHK(hipGetLastError());
    sap_stats local;
    memset(&local, 0, sizeof(local));
    const Params P = toParams(params);
-   RCCHK(beginCall(&b, 1, 1));   // generation 1: the redundancy flags are cleared too
-   RCCHK(runRoundsHost(&b, P, &local));
+   b.redgen = 1;   // the redundancy flags are 0, which no generation is
+   RCCHK(beginCall(&b, 1, 1, P.maxrounds));
+   RCCHK(runRounds(&b, P, &local));
    local.result = c->hstatus->cutoff ? SAP_CUTOFF : (c->hstatus->nchg > 0 ? SAP_REDUCEDDOM : SAP_DIDNOTFIND);
    if( local.result != SAP_CUTOFF )
    {
