@@ -3193,14 +3193,14 @@ __global__ __launch_bounds__(SAP_STAT_SLOTS) void k_round_begin(Vec V, int32_t m
 // generation 1 clears the first nclear flags (those of every vector) first.  With begin set
 // (a launch of one workgroup, nothing enqueued between it and the first round) it also does
 // the first round's k_round_begin, whose stamps were just cleared, saving that launch.
-__global__ void k_call_reset(Vec V, size_t nclear, int32_t nvec, int32_t firstall, int32_t gen, int32_t begin,
-   int32_t maxrounds)
+// (gi: this thread's index of `step`.)
+__device__ __forceinline__ void resetCall(const Vec& V, size_t nclear, int32_t nvec, int32_t firstall, int32_t gen,
+   int32_t begin, int32_t maxrounds, size_t gi, size_t step)
 {
-   for( size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < nclear; i += (size_t)gridDim.x * blockDim.x )
+   for( size_t i = gi; i < nclear; i += step )
       V.redundant[i] = 0;
-   const size_t gi = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
    const size_t nunits = (size_t)nvec * (size_t)V.nseg;
-   for( size_t u = gi; u < nunits; u += (size_t)gridDim.x * blockDim.x )
+   for( size_t u = gi; u < nunits; u += step )
    {
       V.vcutoff[u] = 0;
       V.vrounds[u] = 0;
@@ -3263,6 +3263,26 @@ __global__ void k_call_reset(Vec V, size_t nclear, int32_t nvec, int32_t firstal
       __syncthreads();
       roundAdvance(V, maxrounds);
    }
+}
+
+__global__ void k_call_reset(Vec V, size_t nclear, int32_t nvec, int32_t firstall, int32_t gen, int32_t begin,
+   int32_t maxrounds)
+{
+   resetCall(V, nclear, nvec, firstall, gen, begin, maxrounds, blockIdx.x * (size_t)blockDim.x + threadIdx.x,
+      (size_t)gridDim.x * blockDim.x);
+}
+
+// start of a call on vector 0 whose bounds wait in mapped host memory: every workgroup takes over
+// its columns, the first one also resets the call (nothing to clear) and may begin its first
+// round; one launch fewer than a reset behind an interleave (with the status riding on k_land, two
+// launches fewer a call: sap_propagate on 2,000 x 5,000 84 -> 80 us)
+__global__ void k_call_start(Vec V, int32_t firstall, int32_t gen, int32_t begin, int32_t maxrounds, const double* lb,
+   const double* ub, int64_t ncols)
+{
+   for( int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < ncols; i += (int64_t)gridDim.x * blockDim.x )
+      V.bnd[i] = make_double2(lb[i], ub[i]);
+   if( blockIdx.x == 0 )
+      resetCall(V, 0, 1, firstall, gen, begin, maxrounds, threadIdx.x, blockDim.x);
 }
 
 // sparse mode: initial worklists hold every row of every vector
@@ -3722,16 +3742,20 @@ __global__ void k_noalloc_begin(Vec V, const double* lb, const double* ub, int64
    }
 }
 
-// the outcome of a call on vector 0, written to mapped host memory after every round group once
-// the call has ended (its done flag, or the stop test the host applies after the group): the
+// the status of a call on vector 0, written to mapped host memory after every round group (hst
+// NULL: not asked for), and its outcome once the call has ended (its done flag, or the stop test the host applies after the group): the
 // bounds (lb NULL: not asked for), and the first histmax entries of the reason history as 32-bit
 // words (hist NULL: none)
-__global__ void k_land(Vec V, int64_t ncols, int32_t maxrounds, double* lb, double* ub, uint32_t* hist, uint32_t histmax)
+__global__ void k_land(Vec V, int64_t ncols, int32_t maxrounds, uint32_t* hst, double* lb, double* ub, uint32_t* hist,
+   uint32_t histmax)
 {
    const Status* st = V.st;
+   const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+   if( hst != NULL )
+      for( int64_t i = i0; i < (int64_t)(sizeof(Status) / 4); i += step )
+         hst[i] = ((const uint32_t*)st)[i];
    if( !st->done && !stopsNext(*st, V.dense != 0, maxrounds) )
       return;
-   const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
    if( hist != NULL )
    {
       const int64_t n = (int64_t)(st->histn < histmax ? st->histn : histmax) * (int64_t)(sizeof(HistRec) / 4);
@@ -3917,6 +3941,8 @@ struct sap_bounds
    Status* dstatus;
    int64_t device_bytes;
    double* stage;   // device staging for host lb/ub (2*ncols)
+   const double* inlb;   // bounds of vector 0 waiting in mapped host memory (device addresses), taken
+   const double* inub;   // over by the next beginCall
    int2* wlmem;     // the worklists and the touched list (V.wl, V.touched)
    int32_t roundbase;
    int32_t graphbroken;   // capture failed once: use the host-driven loop
@@ -5238,7 +5264,8 @@ static void startThreads(std::vector<std::thread>& th, int want, F fn)
 // 87 us.  Longer arrays
 // are copied by the runtime, which reads pageable memory at the link's rate (25 us a MiB),
 // while helper threads look for NaNs.  room: staging the caller needs behind the arrays.
-static int uploadBounds(sap_bounds* b, int32_t v, const double* lb, const double* ub, size_t room = 0)
+// defer: the next beginCall takes the staged arrays over, without a launch of its own.
+static int uploadBounds(sap_bounds* b, int32_t v, const double* lb, const double* ub, size_t room = 0, bool defer = false)
 {
    sap_matrix* m = b->mat;
    sap_context* c = m->ctx;
@@ -5287,8 +5314,14 @@ static int uploadBounds(sap_bounds* b, int32_t v, const double* lb, const double
          return SAP_INVALIDDATA;
    }
    const int32_t v0 = v < 0 ? 0 : v, v1 = v < 0 ? b->nvec : v + 1;
-   for( int32_t q = v0; q < v1; ++q )
-      k_interleave<<<gridFor((size_t)nc), SAP_BLOCK, 0, s>>>(b->V.bnd + (size_t)q * (size_t)nc, dl, du, nc);
+   if( defer && nc <= SAP_RING_COLS )
+   {
+      b->inlb = dl;
+      b->inub = du;
+   }
+   else
+      for( int32_t q = v0; q < v1; ++q )
+         k_interleave<<<gridFor((size_t)nc), SAP_BLOCK, 0, s>>>(b->V.bnd + (size_t)q * (size_t)nc, dl, du, nc);
    HIPCHK(hipGetLastError());
    touchedVectors(b, v);
    return SAP_OKAY;
@@ -5734,12 +5767,10 @@ struct LandSpec
    uint32_t histmax;
 };
 
-static int enqueueLand(sap_bounds* b, const Params& P, const LandSpec* land)
+static int enqueueLand(sap_bounds* b, const Params& P, const LandSpec* land, Status* hst)
 {
-   if( land == NULL )
-      return SAP_OKAY;
-   k_land<<<gridFor((size_t)b->mat->ncols), SAP_BLOCK, 0, b->mat->ctx->stream>>>(b->V, b->mat->ncols, P.maxrounds,
-      land->lb, land->ub, land->hist, land->histmax);
+   k_land<<<gridFor(std::max((size_t)b->mat->ncols, sizeof(Status) / 4)), SAP_BLOCK, 0, b->mat->ctx->stream>>>(b->V,
+      b->mat->ncols, P.maxrounds, (uint32_t*)hst, land->lb, land->ub, land->hist, land->histmax);
    HIPCHK(hipGetLastError());
    return SAP_OKAY;
 }
@@ -5763,7 +5794,7 @@ static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t m
       }
       if( land != NULL )
       {
-         RCCHK(enqueueLand(b, P, land));
+         RCCHK(enqueueLand(b, P, land, NULL));
          HIPCHK(hipStreamSynchronize(b->mat->ctx->stream));
       }
       return SAP_OKAY;
@@ -5805,13 +5836,15 @@ static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t m
             enqueueRound(b, M0, P, L0, s, NULL, NULL);
       else
          HIPCHK(hipGraphLaunch(b->graph[kSchedule[it < 3 ? it - 1 : 2]].exec, s));
-      // the status goes to mapped host memory by a copy kernel on the stream
-      k_copy_words<<<gridFor(sizeof(Status) / 4), SAP_BLOCK, 0, s>>>((uint32_t*)c->hstatusd, (const uint32_t*)b->dstatus,
+      // the status goes to mapped host memory by a copy kernel on the stream, or with the outcome
+      if( land != NULL )
+         RCCHK(enqueueLand(b, P, land, c->hstatusd));
+      else
+         k_copy_words<<<gridFor(sizeof(Status) / 4), SAP_BLOCK, 0, s>>>((uint32_t*)c->hstatusd, (const uint32_t*)b->dstatus,
          sizeof(Status) / 4);
       if( metan > 0 )
          k_pack_meta<<<gridFor((size_t)metan), SAP_BLOCK, 0, s>>>(b->V, metan, (int32_t*)b->hdnd);
       HIPCHK(hipGetLastError());
-      RCCHK(enqueueLand(b, P, land));
       // the end event of the call rides on every group's synchronisation, so that the last
       // one needs no further round trip
       HIPCHK(hipEventRecord(c->ev[1], s));
@@ -5871,7 +5904,16 @@ static int beginCall(sap_bounds* b, int32_t nvec, int32_t firstall, int32_t maxr
    const unsigned grid = gridFor(work);
    const int32_t begin = (maxrounds >= -1 && grid == 1) ? 1 : 0;
    static_assert(SAP_BLOCK == SAP_STAT_SLOTS, "one workgroup of k_call_reset covers the stat slots");
-   k_call_reset<<<grid, SAP_BLOCK, 0, s>>>(b->V, nclear, nvec, firstall, gen, begin, maxrounds);
+   const double *lb = b->inlb, *ub = b->inub;
+   b->inlb = b->inub = NULL;
+   if( lb != NULL && nvec == 1 && nclear == 0 )
+      k_call_start<<<gridFor((size_t)m->ncols), SAP_BLOCK, 0, s>>>(b->V, firstall, gen, begin, maxrounds, lb, ub, m->ncols);
+   else
+   {
+      if( lb != NULL )
+         k_interleave<<<gridFor((size_t)m->ncols), SAP_BLOCK, 0, s>>>(b->V.bnd, lb, ub, m->ncols);
+      k_call_reset<<<grid, SAP_BLOCK, 0, s>>>(b->V, nclear, nvec, firstall, gen, begin, maxrounds);
+   }
    HIPCHK(hipGetLastError());
    b->redgen = gen;
    b->begun = begin;
@@ -6021,7 +6063,7 @@ int sap_propagate_reasons(sap_matrix* m, const sap_params* params, double* lb, d
    sap_stats local;
    for( int attempt = 0;; ++attempt )
    {
-      RCCHK(uploadBounds(b, 0, lb, ub, 2 * nb + SAP_LAND_HIST * sizeof(HistRec)));
+      RCCHK(uploadBounds(b, 0, lb, ub, 2 * nb + SAP_LAND_HIST * sizeof(HistRec), true));
       if( small )
       {
          land.lb = (double*)(c->ringd + 2 * nb);
@@ -6132,7 +6174,7 @@ int sap_propagate(sap_matrix* m, const sap_params* params, double* lb, double* u
    sap_bounds* b = m->single;
    const size_t nb = 8 * (size_t)m->ncols;
    const bool small = m->ncols <= SAP_RING_COLS;
-   RCCHK(uploadBounds(b, 0, lb, ub, 2 * nb));
+   RCCHK(uploadBounds(b, 0, lb, ub, 2 * nb, true));
    sap_stats local;
    memset(&local, 0, sizeof(local));
    LandSpec land;

@@ -69,3 +69,25 @@ def test_calls(gpu_ctx, ncols):
     assert rnd[0] == orr["rounds"]
     assert np.array_equal(lb, np.concatenate([ol, ol, none.lb])) and np.array_equal(ub, np.concatenate([ou, ou, none.ub]))
     packed.close()
+
+
+def test_many_calls(gpu_ctx):
+    # more calls than the redundant-row generations (255) on one matrix: the calls that start the
+    # generations again take the bounds over apart from the reset
+    inst = sa.gen_covering_packing(40, 60, 8, seed=3)
+    mat = sa.Matrix(gpu_ctx, inst)
+    om = orc.OMatrix.from_instance(inst)
+    rng = np.random.default_rng(4)
+    print("[case] 520 calls on one matrix", flush=True)
+    for _ in range(520):
+        lb, ub = inst.lb.copy(), inst.ub.copy()
+        j = rng.choice(60, size=4, replace=False)
+        lb[j[:2]], ub[j[2:]] = 1.0, 0.0
+        ol, ou, orr = orc.propagate_jacobi(om, lb, ub)
+        gl, gu, st = mat.propagate(lb, ub)
+        assert (st["result"] == sa.SAP_CUTOFF) == bool(orr["cutoff"])
+        if not orr["cutoff"]:
+            assert np.array_equal(gl, ol) and np.array_equal(gu, ou) and st["nchgbds"] == orr["nchgbds"]
+        else:
+            assert np.array_equal(gl, lb) and np.array_equal(gu, ub)
+    mat.close()
