@@ -535,10 +535,42 @@ struct MarkShared
    uint32_t base[SAP_NBINS];     // their first worklist position
 };
 
-// rows marked for round `first` and appended to its worklists by a whole workgroup: thread t's
-// column has the rows rowidx[beg .. beg + len) in vector v (len 0: no column).  The rows are
-// numbered across the workgroup, so that every thread takes the next one whatever the column
-// lengths; SAP_MARK_ROWS per thread and pass are tagged first, then the fresh ones counted per
+// the rows of a workgroup's columns, numbered across the workgroup, so that every thread takes the
+// next one whatever the column lengths: thread t's column has the rows rowidx[beg .. beg + len)
+// in vector v (len 0: no column).  Returns their total; barriers inside.
+__device__ __forceinline__ int64_t numberRows(MarkShared& S, int64_t beg, int64_t len, int32_t v)
+{
+   const int t = (int)threadIdx.x;
+   int64_t total;
+   const int64_t mine = blockScan(len, S.wsum, total);
+   S.off[t] = mine;
+   S.beg[t] = beg;
+   S.vec[t] = v;
+   if( t == 0 )
+      S.off[SAP_BLOCK] = total;
+   __syncthreads();
+   return total;
+}
+
+// row and vector of number f < total
+__device__ __forceinline__ void numberedRow(const Mat& M, const MarkShared& S, int64_t f, int32_t& row, int32_t& v)
+{
+   // the column of row f: the largest k with off[k] <= f, which has off[k + 1] > f
+   int lo = 0, hi = SAP_BLOCK - 1;
+   while( lo < hi )
+   {
+      const int mid = (lo + hi + 1) >> 1;
+      if( S.off[mid] <= f )
+         lo = mid;
+      else
+         hi = mid - 1;
+   }
+   v = S.vec[lo];
+   row = M.rowidx[S.beg[lo] + (f - S.off[lo])];
+}
+
+// rows marked for round `first` and appended to its worklists by a whole workgroup (numberRows);
+// SAP_MARK_ROWS per thread and pass are tagged first, then the fresh ones counted per
 // length bin in LDS and appended with one global atomic per bin.  What bounds it is the chain
 // of a pass (row index, tag, bin, LDS count, append), so a pass is long.  skipred: rows that
 // are locally redundant are not marked.
@@ -584,14 +616,7 @@ __device__ __forceinline__ void blockMark(const Mat& M, const Vec& V, MarkShared
    const int t = (int)threadIdx.x;
    const int par = first & 1;
    const uint8_t gen = redGen(V);
-   int64_t total;
-   const int64_t mine = blockScan(len, S.wsum, total);
-   S.off[t] = mine;
-   S.beg[t] = beg;
-   S.vec[t] = v;
-   if( t == 0 )
-      S.off[SAP_BLOCK] = total;
-   __syncthreads();
+   const int64_t total = numberRows(S, beg, len, v);
    // passes are workgroup-uniform: total is the same in every thread
    for( int64_t f0 = 0; f0 < total; f0 += SAP_MARK_ROWS * SAP_BLOCK )
    {
@@ -608,18 +633,8 @@ __device__ __forceinline__ void blockMark(const Mat& M, const Vec& V, MarkShared
          item[k] = make_int2(0, 0);
          if( f < total )
          {
-            // the column of row f: the largest k with off[k] <= f, which has off[k + 1] > f
-            int lo = 0, hi = SAP_BLOCK - 1;
-            while( lo < hi )
-            {
-               const int mid = (lo + hi + 1) >> 1;
-               if( S.off[mid] <= f )
-                  lo = mid;
-               else
-                  hi = mid - 1;
-            }
-            const int32_t rv = S.vec[lo];
-            const int32_t row = M.rowidx[S.beg[lo] + (f - S.off[lo])];
+            int32_t rv, row;
+            numberedRow(M, S, f, row, rv);
             const size_t rflat = (size_t)rv * (size_t)M.nrows + (size_t)row;
             if( !skipred || V.redundant[rflat] != gen )
             {
@@ -648,6 +663,29 @@ __device__ __forceinline__ void blockMark(const Mat& M, const Vec& V, MarkShared
       for( int k = 0; k < SAP_MARK_ROWS; ++k )
          if( bin[k] >= 0 && S.base[bin[k]] + pos[k] < V.listcap )
             V.wl[par][bin[k]][S.base[bin[k]] + pos[k]] = item[k];
+   }
+   __syncthreads();   // S is rewritten by the next columns
+}
+
+// the same rows marked by their tags alone, dense mode (redundant ones too: the sweep skips them);
+// the vector's pending round is set once per column.  A thread that walked its own column was a
+// serial chain over the column's rows: the overlay of one column of 40,000 rows took 5,750 us
+// in a node call that takes 230 us
+__device__ __forceinline__ void blockTag(const Mat& M, const Vec& V, MarkShared& S, int64_t beg, int64_t len, int32_t v,
+   int32_t first, bool& any)
+{
+   const int64_t total = numberRows(S, beg, len, v);
+   if( len > 0 )
+   {
+      if( V.vpend[v] != first )
+         V.vpend[v] = first;   // every writer of this round stores the same value
+      any = true;
+   }
+   for( int64_t f = (int)threadIdx.x; f < total; f += SAP_BLOCK )
+   {
+      int32_t rv, row;
+      numberedRow(M, S, f, row, rv);
+      V.rowmark[(size_t)rv * (size_t)M.nrows + (size_t)row] = first;
    }
    __syncthreads();   // S is rewritten by the next columns
 }
@@ -3403,7 +3441,7 @@ __device__ __forceinline__ void slotMarkRow(const Mat& M, const Vec& V, Status* 
 // fixpoint), or every row (grid: rows per slot in x, slots in y).  The overlay entries of all
 // slots (ovptr[0] = 0 .. ovptr[n]) are taken `chunk` at a time over a one-dimensional grid,
 // each thread finding its slot by binary search in ovptr, and their rows are marked and listed
-// by the workgroup (blockMark).  listed: dense mode's flag of this round after the call (1
+// (blockMark) or marked (blockTag) by the workgroup.  listed: dense mode's flag of this round after the call (1
 // also lists, 0 tags alone suffice to mark; -1 as 1, but leaves the flag, which an earlier
 // marking for the same round may have cleared).  Launched with SAP_BLOCK threads.
 __global__ void __launch_bounds__(SAP_BLOCK) k_slot_mark(Mat M, Vec V, const int32_t* slots, int32_t n,
@@ -3454,8 +3492,7 @@ __global__ void __launch_bounds__(SAP_BLOCK) k_slot_mark(Mat M, Vec V, const int
          if( !V.dense || listed != 0 )
             blockMark(M, V, S, beg, len, v, first, false, any);
          else
-            for( int64_t q = beg; q < beg + len; ++q )
-               slotMarkRow(M, V, st, v, M.rowidx[q], first, par, any);
+            blockTag(M, V, S, beg, len, v, first, any);
       }
    }
    if( V.dense && blockIdx.x == 0 && blockIdx.y == 0 && t == 0 && listed >= 0 )

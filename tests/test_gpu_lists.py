@@ -2,6 +2,8 @@
 of very high degree is fixed, so that few changed columns mark many rows (more than a row list
 holds) and these touch many columns (more than the touched list holds).  Against the oracle's
 Jacobi twin: bit-exact bounds, verdicts, rounds and counts."""
+import time
+
 import numpy as np
 import pytest
 
@@ -67,6 +69,44 @@ def test_lists_end_from_overlays(gpu_ctx, n):
         a, b, c = out["chgptr"][1:].tolist()
         assert np.array_equal(out["chgcol"][:a], np.arange(1, n + 2)) and np.all(out["chgub"][:a] == 0.0)
         assert out["chgcol"][a:b].tolist() == [0, 4, 6] and np.all(out["chgub"][a:b] == 0.0) and b == c
+    nodes.close()
+    base.close()
+    mat.close()
+
+
+# a dense set that never lists from marking: the rows of the overlay columns are shared out over the
+# workgroup; around one pass of 256 rows, and a column so long that one thread walking it would
+# be a chain of thousands of steps
+@pytest.mark.parametrize("n", [255, 256, 257, 40_000])
+def test_long_overlay_column(gpu_ctx, n):
+    print(f"[case] long overlay column n={n}", flush=True)
+    inst = star(n, force=False)
+    om = orc.OMatrix.from_instance(inst)
+    mat = sa.Matrix(gpu_ctx, inst)
+    base = sa.Bounds(mat, 1)
+    base.upload(inst.lb, inst.ub)
+    nodes = sa.Bounds(mat, 1, sa.SAP_MODE_DENSE)   # at most 21 rows of three to a tile: 1,905 tiles
+    p = sa.default_params(flags=sa.SAP_FLAG_BASE_IS_FIXPOINT)
+    for c, x in (([0], [1.0]), ([2], [1.0]), ([0, 7, n], [0.0, 1.0, 1.0]), ([0, 9], [1.0, 1.0])):
+        out = nodes.propagate_nodes(base, 0, [0, len(c)], c, x, x, params=p, chgcap=n + 64)
+        lb, ub = inst.lb.copy(), inst.ub.copy()
+        lb[c] = ub[c] = x
+        ol, ou, orr = orc.propagate_jacobi(om, lb, ub)
+        assert (out["result"][0] == sa.SAP_CUTOFF) == bool(orr["cutoff"]) == (c == [0, 9])
+        if not orr["cutoff"]:
+            lb[out["chgcol"]], ub[out["chgcol"]] = out["chglb"], out["chgub"]
+            assert np.array_equal(lb, ol) and np.array_equal(ub, ou), c
+    if n == 40_000:
+        # 40,000 tags by 256 threads are 157 steps of under 1 us; a call takes about 100 us without them
+        def best(col):
+            t = []
+            for _ in range(20):
+                t0 = time.perf_counter()
+                nodes.propagate_nodes(base, 0, [0, 1], [col], [0.0], [0.0], params=p, chgcap=64)
+                t.append(time.perf_counter() - t0)
+            return min(t)
+        short, long = best(5), best(0)
+        assert long < 10 * short, (short, long)
     nodes.close()
     base.close()
     mat.close()
