@@ -3,6 +3,8 @@
 (copied out by helper threads), more chunks than there are slots.  Every value comes back as it
 was, a NaN anywhere is refused and changes nothing, and the calls on host arrays agree with the
 oracle's Jacobi twin."""
+import time
+
 import numpy as np
 import pytest
 
@@ -42,6 +44,50 @@ def test_round_trip(gpu_ctx, ncols):
     assert np.array_equal(lb, inst.lb) and np.array_equal(ub, inst.ub)
     b.close()
     mat.close()
+
+
+def boxes(ncols):
+    rng = np.random.default_rng(ncols)
+    return sa.Instance(rowptr=np.array([0, 1], np.int64), colidx=np.array([ncols - 1], np.int32), vals=np.ones(1),
+                       lhs=np.array([-1e20]), rhs=np.array([1e20]), integral=np.zeros(ncols, np.uint8),
+                       lb=-rng.random(ncols), ub=rng.random(ncols))
+
+
+@pytest.mark.parametrize("ncols", [1, 257, 32_768, 32_769])
+def test_all_vectors(gpu_ctx, ncols):
+    # one pair of arrays into every vector of a set
+    print(f"[case] upload into all vectors ncols={ncols}", flush=True)
+    inst = boxes(ncols)
+    mat = sa.Matrix(gpu_ctx, inst)
+    b = sa.Bounds(mat, 67)
+    b.upload(inst.lb - 2.0, inst.ub + 2.0)
+    b.upload(inst.lb, inst.ub, v=33)
+    for v in (0, 1, 32, 33, 34, 66):
+        off = 0.0 if v == 33 else 2.0
+        lb, ub = b.download(v)
+        assert np.array_equal(lb, inst.lb - off) and np.array_equal(ub, inst.ub + off), v
+    b.close()
+    mat.close()
+
+
+def test_all_vectors_cost(gpu_ctx):
+    # the vectors are filled on the device, whichever way the arrays came there: on the two sides of
+    # the line between the routes an upload into many vectors takes about as long
+    took = []
+    for ncols in (32_000, 33_000):
+        print(f"[case] upload into 256 vectors ncols={ncols}", flush=True)
+        inst = boxes(ncols)
+        mat = sa.Matrix(gpu_ctx, inst)
+        b = sa.Bounds(mat, 256)
+        t = []
+        for _ in range(20):
+            t0 = time.perf_counter()
+            b.upload(inst.lb, inst.ub)
+            t.append(time.perf_counter() - t0)
+        took.append(min(t))
+        b.close()
+        mat.close()
+    assert took[0] < 2.0 * took[1], took
 
 
 @pytest.mark.parametrize("ncols", [32_768, 32_769, 262_145])
