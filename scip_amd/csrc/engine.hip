@@ -52,7 +52,7 @@ using namespace sap;
 #define SAP_MAXLEVELS 40
 #define SAP_ROUND_CAP 10000000
 #define SAP_STAT_SLOTS 256
-#define SAP_CHG_SAMPLE 16   // statistics slots that the marking reads (one cache line)
+#define SAP_CHG_SLOTS 16   // counters of changed bounds, a cache line each
 
 // row-length bins: 0 empty rows; 1..5 at most 4,8,16,32,64 nonzeros (tiles in dense mode,
 // groups of 4,8,16,32,64 lanes in sparse mode); 6 at most 128 nonzeros (tiles of width 2 in
@@ -65,6 +65,12 @@ static const int32_t kBinMaxLen[SAP_NBINS - 2] = { 0, 4, 8, 16, 32, 64, 128 };
 struct alignas(128) Counter
 {
    uint32_t n;
+};
+
+// a statistic that many workgroups add to, likewise
+struct alignas(128) Sum
+{
+   unsigned long long n;
 };
 
 struct Status
@@ -89,8 +95,8 @@ struct Status
    // so workgroups do not serialise on one address); the host sums them after the call
    unsigned long long slot_nnz[SAP_STAT_SLOTS];
    unsigned long long slot_rows[SAP_STAT_SLOTS];
-   unsigned long long slot_chg[SAP_STAT_SLOTS];
-   unsigned long long chgbase;       // the sum of the first SAP_CHG_SAMPLE at the start of the round
+   Sum slot_chg[SAP_CHG_SLOTS];      // changed bounds: few, so that the marking can read them all
+   unsigned long long chgbase;       // their sum at the start of the round
    // sweep launch duration from the constant-rate wall clock: earliest workgroup start and
    // latest workgroup end per slot, folded at the end of the round
    unsigned long long tslot0[SAP_STAT_SLOTS];
@@ -2175,9 +2181,8 @@ __device__ __forceinline__ void sweepBlocks(const Mat& M, const Vec& V, const Pa
    }
 }
 
-// workgroup sum of two per-lane counters, added into the slot of this workgroup
-__device__ __forceinline__ void blockStats(unsigned long long a, unsigned long long b, unsigned long long* slota,
-   unsigned long long* slotb)
+// workgroup sums of two per-lane counters (in thread 0)
+__device__ __forceinline__ void blockSums(unsigned long long& a, unsigned long long& b)
 {
    __shared__ unsigned long long red[2][SAP_BLOCK / SAP_WAVE];
 #pragma unroll
@@ -2194,19 +2199,11 @@ __device__ __forceinline__ void blockStats(unsigned long long a, unsigned long l
    }
    __syncthreads();
    if( threadIdx.x == 0 )
-   {
-      unsigned long long sa = 0, sb = 0;
-      for( int w = 0; w < SAP_BLOCK / SAP_WAVE; ++w )
+      for( int w = 1; w < SAP_BLOCK / SAP_WAVE; ++w )
       {
-         sa += red[0][w];
-         sb += red[1][w];
+         a += red[0][w];
+         b += red[1][w];
       }
-      const int slot = (int)(blockIdx.x & (SAP_STAT_SLOTS - 1));
-      if( sa != 0 )
-         atomicAdd(&slota[slot], sa);
-      if( sb != 0 && slotb != NULL )
-         atomicAdd(&slotb[slot], sb);
-   }
 }
 
 // a listed round's workgroups are shared out over the length bins by the passes that the bins'
@@ -2382,12 +2379,16 @@ __global__ __launch_bounds__(SAP_BLOCK, 4) void k_sweep(Mat M, Vec V, Params P, 
    // remaining queued candidates of this wavefront
    if( Q.count > 0 )
       drainQueue<R>(M, W, P, Q, Q.count, I.round);
-   blockStats(nnzacc, rowsacc, st->slot_nnz, st->slot_rows);   // ends with a barrier
+   blockSums(nnzacc, rowsacc);   // a barrier inside
    if( threadIdx.x == 0 )
    {
+      const int slot = (int)(blockIdx.x & (SAP_STAT_SLOTS - 1));
+      if( nnzacc != 0 )
+         atomicAdd(&st->slot_nnz[slot], nnzacc);
+      if( rowsacc != 0 )
+         atomicAdd(&st->slot_rows[slot], rowsacc);
       if( s_nrecomp != 0 )
          atomicAdd(&st->nrecomp, (unsigned long long)s_nrecomp);
-      const int slot = (int)(blockIdx.x & (SAP_STAT_SLOTS - 1));
       atomicMin(&st->tslot0[slot], tstart);
       atomicMax(&st->tslot1[slot], (unsigned long long)wall_clock64());
    }
@@ -2558,12 +2559,16 @@ __device__ __forceinline__ int columnStep(const Mat& M, const Vec& V, const Para
 // of one workgroup)
 __device__ __forceinline__ void foldStamps(Status* st)
 {
-   __shared__ unsigned long long tmin[SAP_STAT_SLOTS], tmax[SAP_STAT_SLOTS], chg[SAP_CHG_SAMPLE];
+   __shared__ unsigned long long tmin[SAP_STAT_SLOTS], tmax[SAP_STAT_SLOTS];
    const int t = (int)threadIdx.x;
    tmin[t] = st->tslot0[t];
    tmax[t] = st->tslot1[t];
-   if( t < SAP_CHG_SAMPLE )
-      chg[t] = st->slot_chg[t];
+   unsigned long long chg = t < SAP_CHG_SLOTS ? st->slot_chg[t].n : 0;
+#pragma unroll
+   for( int off = 1; off < SAP_CHG_SLOTS; off <<= 1 )
+      chg += (unsigned long long)__shfl_xor((long long)chg, off, SAP_WAVE);
+   if( t == 0 )
+      st->chgbase = chg;   // what the coming round's marking subtracts (markRound)
    st->tslot0[t] = ~0ULL;
    st->tslot1[t] = 0;
    __syncthreads();
@@ -2575,13 +2580,6 @@ __device__ __forceinline__ void foldStamps(Status* st)
          tmax[t] = tmax[t] > tmax[t + w] ? tmax[t] : tmax[t + w];
       }
       __syncthreads();
-   }
-   if( t == 0 )
-   {
-      unsigned long long sum = 0;
-      for( int q = 0; q < SAP_CHG_SAMPLE; ++q )
-         sum += chg[q];
-      st->chgbase = sum;   // what the coming round's marking subtracts (markRound)
    }
    if( t == 0 && tmin[0] != ~0ULL && tmax[0] >= tmin[0] )
    {
@@ -2665,7 +2663,10 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_columns(Mat M, Vec V, Params P)
          nchg += (unsigned long long)columnStep(M, V, P, t.x, t.y, next);
       }
    }
-   blockStats(nchg, 0, st->slot_chg, NULL);
+   unsigned long long none = 0;
+   blockSums(nchg, none);
+   if( threadIdx.x == 0 && nchg != 0 )
+      atomicAdd(&st->slot_chg[blockIdx.x % SAP_CHG_SLOTS].n, nchg);
 }
 
 // second half of the column step: rows of the columns changed in this round are marked for the
@@ -2685,14 +2686,18 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
 {
    Status* st = V.st;
    const RoundView rv = roundView(V);
-   // changed bounds of this round, estimated from the column step's first statistics slots (its
-   // workgroup w counts in slot w modulo SAP_STAT_SLOTS, and its grid is this one): reading
-   // all of them, with the barriers that takes, cost every scanned round 5-7 us
+   // changed bounds of this round, on SAP_CHG_SLOTS lines read together with the round's fields
+   // (as many slots as the sweep's statistics have took barriers to sum: 5-7 us of every scanned
+   // round; a sample of them mistook changes that cluster by column: 282 -> 490 us a call of
+   // 65,000 rows whose changed columns come last)
    unsigned long long changed = 0;
+   if( V.listper > 0 )
+   {
 #pragma unroll
-   for( int q = 0; q < SAP_CHG_SAMPLE; ++q )
-      changed += st->slot_chg[q];
-   changed -= st->chgbase;
+      for( int q = 0; q < SAP_CHG_SLOTS; ++q )
+         changed += st->slot_chg[q].n;
+      changed -= st->chgbase;
+   }
    if( rv.done || (V.single && rv.cutoff) )
       return;
    __shared__ MarkShared S;
@@ -2736,9 +2741,7 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
    }
    else
    {
-      const unsigned used = gridDim.x < SAP_STAT_SLOTS ? gridDim.x : SAP_STAT_SLOTS;
-      const unsigned scale = used > SAP_CHG_SAMPLE ? used / SAP_CHG_SAMPLE : 1;
-      list = V.listper > 0 && changed * scale <= (unsigned long long)V.listper * (unsigned long long)V.nvec;
+      list = V.listper > 0 && changed <= (unsigned long long)V.listper * (unsigned long long)V.nvec;
       const size_t n = (size_t)V.nvec * (size_t)M.ncols;
       if( !list )
       {
@@ -3287,7 +3290,8 @@ __device__ __forceinline__ void resetCall(const Vec& V, size_t nclear, int32_t n
    {
       V.st->slot_nnz[gi] = 0;
       V.st->slot_rows[gi] = 0;
-      V.st->slot_chg[gi] = 0;
+      if( gi < SAP_CHG_SLOTS )
+         V.st->slot_chg[gi].n = 0;
       V.st->tslot0[gi] = ~0ULL;
       V.st->tslot1[gi] = 0;
    }
@@ -3510,7 +3514,8 @@ __global__ void k_step_begin(Vec V)
    {
       st->slot_nnz[t] = 0;
       st->slot_rows[t] = 0;
-      st->slot_chg[t] = 0;
+      if( t < SAP_CHG_SLOTS )
+         st->slot_chg[t].n = 0;
       st->tslot0[t] = ~0ULL;
       st->tslot1[t] = 0;
    }
@@ -5605,8 +5610,9 @@ static void foldStats(sap_context* c)
    {
       a += h->slot_nnz[q];
       r += h->slot_rows[q];
-      g += h->slot_chg[q];
    }
+   for( int q = 0; q < SAP_CHG_SLOTS; ++q )
+      g += h->slot_chg[q].n;
    h->nnz_swept = a;
    h->rows_swept = r;
    h->nchg = g;
@@ -7483,8 +7489,9 @@ int sap_slots_wait(sap_bounds* b, int32_t* nfinished, int32_t* finished, sap_sta
       {
          a += h->slot_nnz[q];
          r += h->slot_rows[q];
-         g += h->slot_chg[q];
       }
+      for( int q = 0; q < SAP_CHG_SLOTS; ++q )
+         g += h->slot_chg[q].n;
       float ms = 0.0f;
       HIPCHK(hipEventElapsedTime(&ms, b->evs[0], b->evs[1]));
       memset(stats, 0, sizeof(*stats));
