@@ -14,19 +14,28 @@ from tests.test_zz_no_alloc import DeviceArray
 pytestmark = pytest.mark.gpu
 
 
-def star(n, force):
+# a tile of the sweep holds at most 256 nonzeros, and only sets of many tiles list rows: with these
+# rows beside them (64 of 1,000 further columns each, never binding) 4,375 tiles at least
+IDLE = 17_500
+
+
+def star(n, force, idle=0):
     """x0 + y_i + y_(i+1) <= 1 over binaries for i = 1..n, then (force) the row x0 >= 1: its round
-    changes one column, whose n rows then fix every y."""
-    rows = n + (1 if force else 0)
-    rowptr = np.concatenate([3 * np.arange(n + 1), [3 * n + 1] if force else []]).astype(np.int64)
+    changes one column, whose n rows then fix every y; then rows that never change anything."""
+    rows = n + (1 if force else 0) + idle
+    length = np.concatenate([np.full(n, 3), [1] if force else [], np.full(idle, 64)]).astype(np.int64)
+    rowptr = np.concatenate([[0], np.cumsum(length)]).astype(np.int64)
     i = np.arange(1, n + 1)
     colidx = np.stack([np.zeros(n, np.int64), i, i + 1], 1).reshape(-1)
-    colidx = np.concatenate([colidx, [0]] if force else [colidx]).astype(np.int32)
+    rest = n + 2 + np.sort((np.arange(64) * 15 + np.arange(idle)[:, None]) % 1000, axis=1).reshape(-1)
+    colidx = np.concatenate([colidx, [0] if force else [], rest]).astype(np.int32)
     lhs, rhs = np.full(rows, -1e20), np.full(rows, 1.0)
     if force:
         lhs[n], rhs[n] = 1.0, 1e20
+    rhs[rows - idle:] = 100.0
+    cols = n + 2 + (1000 if idle else 0)
     return sa.Instance(rowptr=rowptr, colidx=colidx, vals=np.ones(len(colidx)), lhs=lhs, rhs=rhs,
-                       integral=np.ones(n + 2, dtype=np.uint8), lb=np.zeros(n + 2), ub=np.ones(n + 2))
+                       integral=np.ones(cols, dtype=np.uint8), lb=np.zeros(cols), ub=np.ones(cols))
 
 
 # rows of one length bin and touched columns: within every list; beyond the no-allocation
@@ -34,7 +43,7 @@ def star(n, force):
 @pytest.mark.parametrize("n", [32_700, 33_000, 70_000, 131_000, 135_000])
 def test_lists_end(gpu_ctx, n):
     print(f"[case] lists n={n}", flush=True)
-    inst = star(n, force=True)
+    inst = star(n, force=True, idle=IDLE)
     ol, ou, orr = orc.propagate_jacobi(orc.OMatrix.from_instance(inst), inst.lb, inst.ub)
     assert not orr["cutoff"] and orr["rounds"] == 3 and orr["nchgbds"] == n + 2
     mat = sa.Matrix(gpu_ctx, inst)
@@ -55,7 +64,7 @@ def test_lists_end_from_overlays(gpu_ctx, n):
     # the same rows marked by a node's overlay, next to a node with a single marked row pair and
     # one that is cut off, in one dense set; then again on the same set
     print(f"[case] lists from overlays n={n}", flush=True)
-    inst = star(n, force=False)
+    inst = star(n, force=False, idle=IDLE)
     mat = sa.Matrix(gpu_ctx, inst)
     base = sa.Bounds(mat, 1)
     base.upload(inst.lb, inst.ub)
@@ -115,7 +124,7 @@ def test_long_overlay_column(gpu_ctx, n):
 def test_clustered_changes(gpu_ctx):
     # which rounds are listed follows from how many columns changed, not from where they are: a system
     # with its changing columns first, last and spread, and the time of a call on each
-    inst = sa.gen_mixed(65_000, 65_000, seed=11, planted=True)
+    inst = sa.gen_mixed(130_000, 65_000, seed=11, planted=True)   # 65,536 columns: one workgroup a counter
     mat = sa.Matrix(gpu_ctx, inst)
     lb, ub, st = mat.propagate()
     mat.close()
