@@ -2608,9 +2608,9 @@ __host__ __device__ __forceinline__ bool stopsNext(const Status& st, bool dense,
    return !more || st.cutoff || (!st.cont && maxrounds >= 0 && st.rlocal >= maxrounds);
 }
 
-// mark the rows of a changed column for the next round (eventExecLinear marks them) by their
-// tags alone
-__device__ __forceinline__ void markColumn(const Mat& M, const Vec& V, int32_t j, int32_t v, int32_t next,
+// mark the rows of a changed column, rowidx[beg .. end), for the next round (eventExecLinear marks
+// them) by their tags alone
+__device__ __forceinline__ void markColumn(const Mat& M, const Vec& V, int64_t beg, int64_t end, int32_t v, int32_t next,
    bool& anymarked)
 {
    // Round tags are stored without being read first, also on locally redundant rows, which
@@ -2618,7 +2618,7 @@ __device__ __forceinline__ void markColumn(const Mat& M, const Vec& V, int32_t j
    // round (its pending round, the round's "any row marked") reads the redundant flags
    // only until such a row is known.
    bool known = V.vpend[v] == next;
-   for( int64_t q = M.colptr[j]; q < M.colptr[j + 1]; ++q )
+   for( int64_t q = beg; q < end; ++q )
    {
       const size_t rflat = (size_t)v * (size_t)M.nrows + (size_t)M.rowidx[q];
       V.rowmark[rflat] = next;
@@ -2682,28 +2682,64 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_columns(Mat M, Vec V, Params P)
 #define SAP_MARK_BLOCKS 512   // workgroups that list rows (an atomic per workgroup and length bin)
 #define SAP_MARK_FLATS (4 * SAP_BLOCK)
 
+// the rows of column flat (of all vectors' columns), beg .. end of rowidx, and its vector; none when
+// its unit was cut off
+__device__ __forceinline__ void changedRows(const Mat& M, const Vec& V, size_t flat, int64_t& beg, int64_t& end,
+   int32_t& v)
+{
+   v = (int32_t)(flat / (size_t)M.ncols);
+   const int32_t j = (int32_t)(flat - (size_t)v * (size_t)M.ncols);
+   beg = M.colptr[j];
+   end = V.vcutoff[unitOfCol(M, v, j)] == 0 ? M.colptr[j + 1] : beg;
+}
+
+// scanned marking of the columns flat0, flat0 + the grid's threads, ... by their tags; the first
+// one's rows are known
+__device__ __forceinline__ void markTags(const Mat& M, const Vec& V, size_t flat0, size_t n, int64_t beg, int64_t end,
+   int32_t v, int32_t round, bool& anymarked)
+{
+   if( beg < end )
+      markColumn(M, V, beg, end, v, round + 1, anymarked);
+   for( size_t flat = flat0 + (size_t)gridDim.x * SAP_BLOCK; flat < n; flat += (size_t)gridDim.x * SAP_BLOCK )
+   {
+      if( V.chgtag[flat] != round )
+         continue;
+      changedRows(M, V, flat, beg, end, v);
+      markColumn(M, V, beg, end, v, round + 1, anymarked);
+   }
+}
+
+__device__ __forceinline__ void noteMarked(Status* st, int32_t next, bool anymarked)
+{
+   if( __ballot(anymarked) != 0 && ((int)threadIdx.x & (SAP_WAVE - 1)) == 0 && st->anymark[next & 1] == 0 )
+      st->anymark[next & 1] = 1;
+}
+
 __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
 {
    Status* st = V.st;
-   const RoundView rv = roundView(V);
-   // changed bounds of this round, on SAP_CHG_SLOTS lines read together with the round's fields
-   // (as many slots as the sweep's statistics have took barriers to sum: 5-7 us of every scanned
-   // round; a sample of them mistook changes that cluster by column: 282 -> 490 us a call of
-   // 65,000 rows whose changed columns come last)
+   const int t = (int)threadIdx.x;
+   // the tag of the thread's first column and the round's changed bounds (SAP_CHG_SLOTS lines that
+   // other XCDs have just added to: 1 us) are asked for together with the round's fields, and the
+   // count is waited for last: a scanned round's marking 10.6 -> 10.4 us (100,000 rows, first
+   // round), 12.2 us when the count came first.  The count is exact: a sample of the columns
+   // mistook changes that cluster by column (282 -> 490 us a call), and a count over as many slots
+   // as the sweep's statistics took barriers, 5-7 us
+   const size_t n = (size_t)V.nvec * (size_t)M.ncols;
+   const size_t flat0 = blockIdx.x * (size_t)SAP_BLOCK + t;
+   int32_t tag0 = 0;
+   if( V.dense && flat0 < n )
+      tag0 = V.chgtag[flat0];
    unsigned long long changed = 0;
-   if( V.listper > 0 )
-   {
-#pragma unroll
-      for( int q = 0; q < SAP_CHG_SLOTS; ++q )
-         changed += st->slot_chg[q].n;
-      changed -= st->chgbase;
-   }
+   if( V.dense && (t & (SAP_WAVE - 1)) < SAP_CHG_SLOTS )
+      changed = st->slot_chg[t & (SAP_WAVE - 1)].n;
+   const unsigned long long before = st->chgbase;
+   const RoundView rv = roundView(V);
    if( rv.done || (V.single && rv.cutoff) )
       return;
    __shared__ MarkShared S;
    __shared__ uint32_t found[SAP_BLOCK + SAP_MARK_FLATS];
    __shared__ uint32_t nfound;
-   const int t = (int)threadIdx.x;
    const int32_t round = rv.round;
    const int32_t next = round + 1;
    bool anymarked = false;
@@ -2725,36 +2761,34 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
             v = e.y;
             chg = V.chgtag[(size_t)v * (size_t)M.ncols + (size_t)j] == round && V.vcutoff[unitOfCol(M, v, j)] == 0;
          }
-         if( !list )
-         {
-            if( chg )
-               markColumn(M, V, j, v, next, anymarked);
-            continue;
-         }
          if( chg )
          {
             beg = M.colptr[j];
             len = M.colptr[j + 1] - beg;
+         }
+         if( !list )
+         {
+            if( chg )
+               markColumn(M, V, beg, beg + len, v, next, anymarked);
+            continue;
          }
          blockMark(M, V, S, beg, len, v, next, true, anymarked);
       }
    }
    else
    {
-      list = V.listper > 0 && changed <= (unsigned long long)V.listper * (unsigned long long)V.nvec;
-      const size_t n = (size_t)V.nvec * (size_t)M.ncols;
+      // the first column's rows are looked up before the count is waited for
+      int64_t beg0 = 0, end0 = 0;
+      int32_t v0 = 0;
+      if( flat0 < n && tag0 == round )
+         changedRows(M, V, flat0, beg0, end0, v0);
+#pragma unroll
+      for( int off = 1; off < SAP_CHG_SLOTS; off <<= 1 )
+         changed += (unsigned long long)__shfl_xor((long long)changed, off, SAP_WAVE);
+      changed = (unsigned long long)__shfl((long long)changed, 0, SAP_WAVE) - before;
+      list = changed <= (unsigned long long)V.listper * (unsigned long long)V.nvec;
       if( !list )
-      {
-         for( size_t flat = blockIdx.x * (size_t)SAP_BLOCK + t; flat < n; flat += (size_t)gridDim.x * SAP_BLOCK )
-         {
-            if( V.chgtag[flat] != round )
-               continue;
-            const int32_t v = (int32_t)(flat / (size_t)M.ncols);
-            const int32_t j = (int32_t)(flat - (size_t)v * (size_t)M.ncols);
-            if( V.vcutoff[unitOfCol(M, v, j)] == 0 )
-               markColumn(M, V, j, v, next, anymarked);
-         }
-      }
+         markTags(M, V, flat0, n, beg0, end0, v0, round, anymarked);
       else
       {
          // the changed columns are collected in LDS and their rows listed SAP_BLOCK columns at
@@ -2806,13 +2840,32 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
    }
    if( V.dense && blockIdx.x == 0 && t == 0 )
       st->listed[next & 1] = list ? 1 : 0;
-   if( __ballot(anymarked) != 0 && (t & (SAP_WAVE - 1)) == 0 && st->anymark[next & 1] == 0 )
-      st->anymark[next & 1] = 1;
+   noteMarked(st, next, anymarked);
 }
 
 __global__ __launch_bounds__(SAP_BLOCK, 8) void k_mark(Mat M, Vec V)
 {
    markRound(M, V);
+}
+
+// ... of a dense set that never lists (listLimits): without the count, the lists and their LDS,
+// which cost each of its rounds 0.5-1 us (50,000 rows, seven rounds: 35.7 -> 33.8 us)
+__global__ __launch_bounds__(SAP_BLOCK) void k_mark_tags(Mat M, Vec V)
+{
+   Status* st = V.st;
+   const size_t n = (size_t)V.nvec * (size_t)M.ncols;
+   const size_t flat0 = blockIdx.x * (size_t)SAP_BLOCK + threadIdx.x;
+   const int32_t tag0 = flat0 < n ? V.chgtag[flat0] : 0;
+   const int32_t round = st->round;
+   if( st->done || (V.single && st->cutoff) )
+      return;
+   int64_t beg0 = 0, end0 = 0;
+   int32_t v0 = 0;
+   if( flat0 < n && tag0 == round )
+      changedRows(M, V, flat0, beg0, end0, v0);
+   bool anymarked = false;
+   markTags(M, V, flat0, n, beg0, end0, v0, round, anymarked);
+   noteMarked(st, round + 1, anymarked);
 }
 
 // reason recording, after the column step: every logged candidate whose key won its column's
@@ -5093,13 +5146,16 @@ static void boundsRelease(sap_bounds* b)
 //   - 1/64 of the rows marked: on the mixed 1M x 1M instance rounds 5-7 (11,807, 324 and 11 rows)
 //     sweep in 57 / 22 / 12 us listed against 79 / 45 / 29 us scanned, and 1/4 listed its round 4,
 //     which then took 214 + 42 us to sweep and to list for against 173 + 10 us;
-//   - sets of few tiles are not listed: a scan visits each wavefront's one tile, while the lists
-//     add their own steps (2,875 x 4,443, 5 rounds: 266 us listed, 254 us scanned).
+//   - sets whose tiles are one to a resident wavefront are not listed: a scan is then one tile a
+//     wavefront, 10-14 us, and a list saves 0-2 us of that and costs its marking 3.5 us (50,000
+//     rows, 2,660 tiles: two rounds listed 7.8 + 6.4 us of marking and 14.0 + 10.4 of sweeps,
+//     scanned 5.1 + 4.5 and 14.2 + 12.7; 80,000 rows, 4,260 tiles: equal; 100,000 rows, 5,325
+//     tiles: the sweeps 15 + 11 instead of 22 + 14 us).
 // 200 strong-branching children of 20,011 rows take 310 us (555-597 us scanned), a node of
 // 148,409 rows among 31 a third of what it took.
 #define SAP_LIST_ROWS ((uint32_t)1 << 17)
 #define SAP_LIST_COLS ((uint32_t)1 << 16)
-#define SAP_LIST_TILES 2048
+#define SAP_LIST_TILES 4096
 
 static void listLimits(const sap_matrix* m, Vec& V)
 {
@@ -5664,7 +5720,10 @@ static void enqueueRound(sap_bounds* b, const Mat& M, const Params& P, const Lay
       k_reason<<<gridFor(2 * (size_t)m->nnz, 4096), SAP_BLOCK, 0, s>>>(b->V);
       k_history<<<gridFor((size_t)m->ncols, 4096), SAP_BLOCK, 0, s>>>(M, b->V);
    }
-   k_mark<<<colgrid, SAP_BLOCK, 0, s>>>(M, b->V);
+   if( b->V.dense && b->V.listper == 0 )
+      k_mark_tags<<<colgrid, SAP_BLOCK, 0, s>>>(M, b->V);
+   else
+      k_mark<<<colgrid, SAP_BLOCK, 0, s>>>(M, b->V);
 }
 
 // ranged-row propagation keeps one check-group flag per (vector, nonzero); allocated on the

@@ -158,3 +158,28 @@ def test_clustered_changes(gpu_ctx):
         mat.close()
     # the same rows are swept in the same rounds; what may differ is how the gathers fall into cache lines
     assert max(took["first"], took["last"]) < 1.3 * took["spread"], took
+
+
+# more columns than one pass of the marking takes (2^20), few enough tiles that the set never lists
+@pytest.mark.parametrize("ncols", [1_048_576, 1_048_577, 1_100_003])
+def test_many_columns(gpu_ctx, ncols):
+    print(f"[case] many columns ncols={ncols}", flush=True)
+    part = sa.gen_mixed(3000, 3000, seed=5, planted=True)
+    at = np.linspace(0, ncols - 1, 3000).astype(np.int64)
+    whole = {}
+    for k, fill in (("lb", 0.0), ("ub", 1.0), ("integral", 0)):
+        whole[k] = np.full(ncols, fill, dtype=getattr(part, k).dtype)
+        whole[k][at] = getattr(part, k)
+    inst = sa.Instance(rowptr=part.rowptr, colidx=at[part.colidx].astype(np.int32), vals=part.vals, lhs=part.lhs,
+                       rhs=part.rhs, **whole)
+    ol, ou, orr = orc.propagate_jacobi(orc.OMatrix.from_instance(inst), inst.lb, inst.ub)
+    assert not orr["cutoff"] and orr["rounds"] >= 3
+    mat = sa.Matrix(gpu_ctx, inst)
+    b = sa.Bounds(mat, 1, sa.SAP_MODE_DENSE)
+    b.upload(inst.lb, inst.ub)
+    st = b.propagate()
+    gl, gu = b.download()
+    assert np.array_equal(gl, ol) and np.array_equal(gu, ou)
+    assert (st["rounds"], st["nchgbds"], st["rows_swept"]) == (orr["rounds"], orr["nchgbds"], orr["rows_swept"])
+    b.close()
+    mat.close()
