@@ -241,7 +241,8 @@ struct HistRec
 struct Layout
 {
    int32_t blockstart[SAP_NKINDS + 1];
-   int32_t longfirst;   // the workgroups start in reverse order: the longest rows' before the tiles'
+   int32_t longfirst;   // the kinds start in reverse order: the longest rows' workgroups before the tiles'
+   int32_t tilesdown;   // ... and the tiles' in descending order
 };
 
 #define KEY_NEG_INF ((long long)0x800FFFFFFFFFFFFFLL)   // dkey(-inf)
@@ -2270,8 +2271,10 @@ __global__ __launch_bounds__(SAP_BLOCK, 4) void k_sweep(Mat M, Vec V, Params P, 
          return;   // a workgroup that only listed rounds use
       while( kind < SAP_NKINDS - 1 && blk >= L.blockstart[kind + 1] )
          ++kind;
-      lblock = blk - L.blockstart[kind];
       nblocks = L.blockstart[kind + 1] - L.blockstart[kind];
+      lblock = blk - L.blockstart[kind];
+      if( L.longfirst && !(kind == 0 && L.tilesdown) )
+         lblock = nblocks - 1 - lblock;
    }
    else if( !listShare(M, *st, I.round & 1, kind, lblock, nblocks) )
       return;
@@ -5575,8 +5578,11 @@ static Layout makeLayout(const sap_bounds* b)
    static const int kCap[SAP_NKINDS] = { 4096, 2048, 2048, 2048, 2048, 2048, 2048, 2048, 2048, 1024 };
    const int tb = m->tuning.tilebins, rb = m->tuning.rowbins;
    size_t blocks[SAP_NKINDS], units[SAP_NKINDS], all = 0, sum = 0;
-   // rough time of an item against a tile's 4, per wavefront (a row of kind 9 takes four)
+   // rough time of an item against a tile's 4, per wavefront (kinds 1-6: of a wavefront's rows; a row
+   // of kind 9 takes four wavefronts, 64 when only rows of more than 1,024 nonzeros are of that
+   // kind and less when shorter ones are)
    static const int kUnits[SAP_NKINDS] = { 4, 4, 4, 4, 4, 4, 4, 3, 5, 64 };
+   const int kind9 = std::max(16, std::min(64, m->tuning.longrow / 16));
    for( int q = 0; q < SAP_NKINDS; ++q )
    {
       const int bin = q - 1;
@@ -5591,7 +5597,7 @@ static Layout makeLayout(const sap_bounds* b)
       blocks[q] = (items + per - 1) / per;
       const size_t cap = std::max<size_t>(64, (size_t)kCap[q] * (size_t)m->tuning.capscale / 100);
       blocks[q] = std::min(blocks[q], cap);
-      units[q] = q >= 1 && q <= 6 ? 0 : items * (size_t)kUnits[q];
+      units[q] = items * (size_t)(q == 9 ? kind9 : kUnits[q]) / (size_t)(q >= 1 && q <= 6 ? per / (SAP_BLOCK / SAP_WAVE) : 1);
       all += units[q];
       sum += blocks[q];
    }
@@ -5599,16 +5605,22 @@ static Layout makeLayout(const sap_bounds* b)
    // fill the device, the wavefronts of the long rows start as the first tiles end, and their
    // chain of 12-14 us is the tail of every scanned round.  With few tiles per wavefront the
    // long rows therefore start first, in a share of the places that follows their work, and the
-   // tiles take the rest: the four scanned sweeps of 100k rows (1.3 tiles per wavefront) 52 / 49
-   // / 45 / 41 -> 46 / 42 / 38 / 32 us, the first four of 300k rows (3.8) 94 / 98 / 93 / 79 -> 99 /
-   // 91 / 84 / 68 us.  With many (1M rows, 12.7) the places cost the tiles more than the tail:
-   // 280 -> 288 us.
+   // tiles take the rest.  Scanned sweeps of a call, tiles first / long rows first: 80,000 rows
+   // (1.15 tiles per wavefront) 174 / 149 us, 100,000 (1.45) 189 / 161 us, 200,000 (2.9) 278 / 252
+   // us, 300,000 (4.3) 377 / 337 us, 500,000 (7.3) 532 / 509 us.  Tiles that do not fill the device
+   // leave the long rows places anyway (70,000 rows: 139 us, 159 us when these took a share), and
+   // with many per wavefront (1M rows, 12.7) the places cost the tiles more than the tail.
+   // The tiles' workgroups start in ascending order, those with one tile more than the others first:
+   // in descending order that tile was the tail (first sweep of 80,000 rows 45 instead of 37 us, of
+   // 300,000 rows 95 instead of 83 us).  Where nearly all have it, descending order measured
+   // better, for a reason not found (130,000 rows, 1.9 tiles: 199 us ascending, 189 us descending;
+   // 200,000 rows, 2.9: 261 and 252 us), so that remains above 4/5 of the wavefronts.
    const size_t res = (size_t)std::max(m->ctx->resident, 0);
-   L.longfirst = 0;
+   L.longfirst = L.tilesdown = 0;
    if( b->V.dense && res > 0 && blocks[0] > 0 )
    {
       size_t room = res;
-      if( sum > res && units[0] / (size_t)kUnits[0] <= 8 * res * (SAP_BLOCK / SAP_WAVE) )
+      if( blocks[0] >= res && units[0] / (size_t)kUnits[0] <= 8 * res * (SAP_BLOCK / SAP_WAVE) )
       {
          size_t others = 0;
          for( int q = 1; q < SAP_NKINDS; ++q )
@@ -5619,6 +5631,8 @@ static Layout makeLayout(const sap_bounds* b)
          }
          room = std::max(res / 2, others < res ? res - others : 0);
          L.longfirst = 1;
+         const size_t tiles = units[0] / (size_t)kUnits[0], waves = room * (SAP_BLOCK / SAP_WAVE);
+         L.tilesdown = 5 * (tiles % waves) > 4 * waves ? 1 : 0;
       }
       blocks[0] = std::min(blocks[0], room);
    }

@@ -12,10 +12,9 @@ pytestmark = pytest.mark.gpu
 LENGTHS = [65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 319, 511, 512, 513, 767, 1023, 1024, 1025, 1280, 2047, 2049, 4100]
 
 
-def long_instance(seed, extra):
-    """Two rows of every length and `extra` short ones over 5,000 columns, planted."""
+def long_instance(seed, extra, n):
+    """Two rows of every length and `extra` short ones over n columns, planted."""
     rng = np.random.default_rng(seed)
-    n = 5000
     integral = (rng.random(n) < 0.4).astype(np.uint8)
     lb = np.where(integral, 0.0, -1e4 * rng.random(n))
     ub = np.where(integral, rng.integers(1, 1000, size=n).astype(float), 1e4 * rng.random(n))
@@ -32,12 +31,23 @@ def long_instance(seed, extra):
     return sa.Instance(rowptr=ptr, colidx=col, vals=val, lhs=act - side, rhs=act + side, integral=integral, lb=lb, ub=ub)
 
 
-# 60 short rows: few tiles; 40,000: more workgroups than the device holds, so the long rows' start first
-@pytest.mark.parametrize("extra", [60, 40_000])
+# 60 and 40,000 short rows: the device holds every workgroup at once.  112,000 and 160,000: the tiles
+# alone fill it (1,024 workgroups of four tiles), so the long rows' workgroups start first, with
+# the tiles' in ascending and in descending order (1.3 and 1.9 tiles per wavefront); late rounds
+# of these are listed (over 4,096 tiles, columns of low degree)
+@pytest.mark.parametrize("extra", [60, 40_000, 112_000, 160_000])
 @pytest.mark.parametrize("longrow", [1024, 64])
 def test_long_rows(gpu_ctx, extra, longrow):
     print(f"[case] long rows extra={extra} longrow={longrow}", flush=True)
-    inst = long_instance(7 + extra, extra)
+    inst = long_instance(7 + extra, extra, 5000 if extra <= 40_000 else 100_000)
+    # lanes of four nonzeros, packed nearly without gaps into tiles of 64; 980 to 1,010 of the
+    # workgroups are the tiles'
+    length = np.diff(inst.rowptr)
+    tiles = np.sum((length[length <= 64] + 3) // 4) / 64
+    if extra == 112_000:
+        assert tiles > 4 * 1024 and tiles / (4 * 980) < 1.7
+    if extra == 160_000:
+        assert 1.8 < tiles / (4 * 1010) and tiles / (4 * 980) < 1.95
     om = orc.OMatrix.from_instance(inst)
     ol, ou, orr = orc.propagate_jacobi(om, inst.lb, inst.ub)
     assert not orr["cutoff"] and orr["rounds"] >= 3
