@@ -17,6 +17,11 @@
  *     except the opaque handles, which have matching *_free functions.
  *   - One sap_context per SCIP instance (SCIP* is single-threaded); a context owns one
  *     HIP stream.  Calls on different contexts may run concurrently.
+ *   - sap_propagate, sap_propagate_reasons, sap_propagate_packed and sap_bounds_upload/_download
+ *     with more than 32,768 columns start up to 4 helper threads, at most one fewer than the CPUs
+ *     the calling thread may run on, to look through and copy the host arrays; they have ended
+ *     when the call returns, and yield while they wait for the device.  On a host shared by many
+ *     processes, confine each (sched_setaffinity); with one CPU no thread is started.
  *   - Arithmetic is IEEE FP64 throughout.
  */
 #ifndef SCIP_AMD_PROP_H

@@ -28,6 +28,7 @@
 // canonical tree, so the result does not depend on the binning.
 #include <hip/hip_runtime.h>
 
+#include <sched.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -3949,6 +3950,7 @@ static __device__ __align__(256) unsigned char g_noalloc_scratch[SAP_NOALLOC_BYT
 // pinned slots; arrays of at most one chunk move in one piece, with the call's own wait
 #define SAP_RING_COLS ((int64_t)32768)
 #define SAP_RING_SLOTS 8
+#define SAP_HELPERS 4   // helper threads of a longer array's transfer, at most
 
 struct sap_context
 {
@@ -5349,21 +5351,36 @@ static bool anyNan(const double* x, int64_t n)
    return bad != 0;
 }
 
-// helper threads of a host array's transfer: as many as can be started, at most `want`
-template <typename F>
-static void startThreads(std::vector<std::thread>& th, int want, F fn)
+// helper threads of a host array's transfer: as many as can be started, at most `want` and one
+// fewer than the CPUs the calling thread may run on (a process confined to one gets none); the
+// calling thread does what no helper takes.  Nothing here throws into the C entry.
+struct Helpers
 {
-   const int hw = (int)std::thread::hardware_concurrency();
-   try
+   std::thread th[SAP_HELPERS];
+   int n = 0;
+
+   template <typename F>
+   void start(int64_t want, F fn)
    {
-      for( int t = 0; t < want && t < hw - 1; ++t )
-         th.emplace_back(fn);
+      cpu_set_t set;
+      int cpus = (int)std::thread::hardware_concurrency();
+      if( sched_getaffinity(0, sizeof(set), &set) == 0 )
+         cpus = CPU_COUNT(&set);
+      try
+      {
+         for( ; n < SAP_HELPERS && n < want && n < cpus - 1; ++n )
+            th[n] = std::thread(fn);
+      }
+      catch( ... )
+      {
+      }
    }
-   catch( ... )
+   void join()
    {
-      // the calling thread does what no helper takes
+      for( int t = 0; t < n; ++t )
+         th[t].join();
    }
-}
+};
 
 // vector v (all for v < 0) of b from host arrays, refused if they hold a NaN.  Up to
 // SAP_RING_COLS columns go through pinned staging and one kernel that reads it, with no wait
@@ -5407,14 +5424,13 @@ static int uploadBounds(sap_bounds* b, int32_t v, const double* lb, const double
                bad = 1;
          }
       };
-      std::vector<std::thread> th;
-      startThreads(th, (int)std::min<int64_t>(3, nc / part), look);
+      Helpers th;
+      th.start(std::min<int64_t>(3, nc / part), look);
       hipError_t e = hipMemcpyAsync(b->stage, lb, sizeof(double) * (size_t)nc, hipMemcpyHostToDevice, s);
       if( e == hipSuccess )
          e = hipMemcpyAsync(b->stage + nc, ub, sizeof(double) * (size_t)nc, hipMemcpyHostToDevice, s);
       look();
-      for( auto& x : th )
-         x.join();
+      th.join();
       if( e != hipSuccess || bad )
          HIPCHK(hipStreamSynchronize(s));   // the caller's arrays are not read after the return
       HIPCHK(e);
@@ -5451,13 +5467,13 @@ static int downloadBounds(sap_context* c, const double2* src, int64_t nc, F take
       if( c->ringev[q] == NULL )
          HIPCHK(hipEventCreateWithFlags(&c->ringev[q], hipEventDisableTiming));
    std::atomic<int64_t> ready(0), next(0);
-   std::vector<std::atomic<int>> copied((size_t)nchunks);
+   std::atomic<int64_t> copied[SAP_RING_SLOTS];   // per slot: 1 + the last chunk copied out of it
    for( auto& x : copied )
       x = 0;
    auto copyOut = [&](int64_t q) {
       const double* l = (const double*)(c->ring + 16 * (size_t)cols * (size_t)(q % slots));
       take(q * cols, std::min(cols, nc - q * cols), l, l + cols);
-      copied[(size_t)q].store(1, std::memory_order_release);
+      copied[q % slots].store(q + 1, std::memory_order_release);
    };
    // ready counts the landed chunks; nchunks + 1 stops the helpers early (an error)
    auto help = [&]() {
@@ -5480,19 +5496,19 @@ static int downloadBounds(sap_context* c, const double2* src, int64_t nc, F take
    hipError_t e = hipSuccess;
    for( int64_t q = 0; q < slots && e == hipSuccess; ++q )
       e = launch(q);
-   std::vector<std::thread> th;
+   Helpers th;
    if( nchunks > 2 )
-      startThreads(th, (int)std::min<int64_t>(4, nchunks / 2), help);
+      th.start(nchunks / 2, help);
    // chunk q lands in its slot once chunk q - slots has been copied out of it; the loop only
    // waits for that when no chunk is in flight
    int64_t launched = slots;
    auto refill = [&](int64_t upto) {
       while( e == hipSuccess && launched < nchunks )
       {
-         const std::atomic<int>& free = copied[(size_t)(launched - slots)];
-         if( free.load(std::memory_order_acquire) == 0 && launched >= upto )
+         const std::atomic<int64_t>& done = copied[launched % slots];
+         if( done.load(std::memory_order_acquire) <= launched - slots && launched >= upto )
             return;
-         while( free.load(std::memory_order_acquire) == 0 )
+         while( done.load(std::memory_order_acquire) <= launched - slots )
             std::this_thread::yield();
          e = launch(launched++);
       }
@@ -5505,16 +5521,15 @@ static int downloadBounds(sap_context* c, const double2* src, int64_t nc, F take
       if( e != hipSuccess )
          break;
       ready.store(q + 1, std::memory_order_release);
-      if( th.empty() )
+      if( th.n == 0 )
          copyOut(q);
       refill(0);
    }
    if( e != hipSuccess )
       ready.store(nchunks + 1, std::memory_order_release);
-   else if( !th.empty() )
+   else if( th.n > 0 )
       help();
-   for( auto& x : th )
-      x.join();
+   th.join();
    if( e != hipSuccess )
       (void)hipStreamSynchronize(s);
    HIPCHK(e);

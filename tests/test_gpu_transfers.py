@@ -3,6 +3,8 @@
 (copied out by helper threads), more chunks than there are slots.  Every value comes back as it
 was, a NaN anywhere is refused and changes nothing, and the calls on host arrays agree with the
 oracle's Jacobi twin."""
+import os
+import threading
 import time
 
 import numpy as np
@@ -137,3 +139,37 @@ def test_many_calls(gpu_ctx):
         else:
             assert np.array_equal(gl, lb) and np.array_equal(gu, ub)
     mat.close()
+
+
+def test_helper_threads_keep_to_the_affinity(gpu_ctx):
+    # a caller confined to one CPU gets no helper threads, and the same values
+    inst = boxes(600_001)
+    mat = sa.Matrix(gpu_ctx, inst)
+    b = sa.Bounds(mat, 1)
+    b.upload(inst.lb, inst.ub)
+    b.download()
+    go, end, wrong = threading.Event(), threading.Event(), []
+
+    def caller():
+        os.sched_setaffinity(0, {min(os.sched_getaffinity(0))})   # this thread only
+        go.wait(60)
+        while not end.is_set():
+            b.upload(inst.lb, inst.ub)
+            lb, ub = b.download()
+            if not (np.array_equal(lb, inst.lb) and np.array_equal(ub, inst.ub)):
+                wrong.append(1)
+
+    print("[case] transfers of a caller on one CPU", flush=True)
+    t = threading.Thread(target=caller)
+    t.start()
+    time.sleep(0.2)
+    threads = len(os.listdir("/proc/self/task"))
+    go.set()
+    until, most = time.perf_counter() + 1.0, 0
+    while time.perf_counter() < until:
+        most = max(most, len(os.listdir("/proc/self/task")))
+    end.set()
+    t.join(60)
+    b.close()
+    mat.close()
+    assert not wrong and most == threads, (most, threads)
