@@ -5759,8 +5759,8 @@ static void enqueueRound(sap_bounds* b, const Mat& M, const Params& P, const Lay
 // first call that asks for it, before any round graph that uses it is captured
 static int ensureRanged(sap_bounds* b, const Params& P)
 {
-   if( !(P.flags & SAP_FLAG_RANGEDROWS) || b->mat->nranged == 0 || b->V.rgflag != NULL )
-      return SAP_OKAY;
+   if( !(P.flags & SAP_FLAG_RANGEDROWS) || rangedRows(toMat(b->mat), P) == 0 || b->V.rgflag != NULL )
+      return SAP_OKAY;   // no ranged step is launched (enqueueRound), or the flags are there
    return devAlloc(&b->V.rgflag, (size_t)b->nvec * (size_t)b->mat->nnz + 1, &b->device_bytes);
 }
 

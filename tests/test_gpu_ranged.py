@@ -1,6 +1,7 @@
 """GPU parity of ranged-row propagation (SAP_FLAG_RANGEDROWS) with the oracle's Jacobi twin
 (rangedrows=1): bit-exact bounds, verdicts and round counts on small gcd-structured systems,
 a large one, the mixed generator, MIPLIB instances, and node batches from a resident base."""
+import ctypes as C
 import os
 
 import numpy as np
@@ -9,6 +10,7 @@ import pytest
 import scip_amd as sa
 from oracle import oracle as orc
 from tests.test_oracle_ranged import ranged_system
+from tests.test_zz_no_alloc import hip
 from tests.util import apply_fixings, random_fixings
 
 pytestmark = pytest.mark.gpu
@@ -84,6 +86,37 @@ def test_coefficients_near_integers(gpu_ctx, eps):
             b.close()
         mat.close()
     assert 0 < cut < 40 and differs > 5   # the ranged step matters in these systems
+
+
+def test_flags_only_for_gcd_rows(gpu_ctx):
+    # the flags of the ranged step (a byte per nonzero and vector) are not allocated for a system
+    # without a row that can hold a gcd group under the default epsilon
+    rng = np.random.default_rng(1350)
+    rows, cols, nvec = 10_000, 1_000, 800
+    col = np.sort(np.argsort(rng.random((rows, 50)), axis=1) + 50 * rng.integers(0, 20, size=(rows, 1)), axis=1)
+    val = rng.uniform(0.1, 0.9, size=col.size)
+    lb, ub = np.zeros(cols), np.full(cols, 4.0)
+    inst = sa.Instance(rowptr=np.arange(0, col.size + 1, 50, dtype=np.int64), colidx=col.reshape(-1).astype(np.int32),
+                       vals=val, lhs=np.full(rows, -1e3), rhs=np.full(rows, 1e3),
+                       integral=np.ones(cols, np.uint8), lb=lb, ub=ub)
+    free, total = C.c_size_t(), C.c_size_t()
+    say("[case] ranged flags of 10,000 rows in 800 vectors")
+    mat = sa.Matrix(gpu_ctx, inst)
+    b = sa.Bounds(mat, nvec)
+    b.upload(lb, ub)
+    b.propagate()   # what any call allocates
+    assert hip().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    before = free.value
+    st = b.propagate(sa.default_params(flags=RANGED))
+    assert st["result"] == sa.SAP_DIDNOTFIND
+    assert hip().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    size = nvec * inst.nnz   # 400 MB
+    assert before - free.value < size // 8
+    # a later call on the same set whose epsilon needs the step on every two-sided row
+    st = b.propagate(sa.default_params(flags=RANGED, epsilon=1e-5))
+    assert st["result"] == sa.SAP_DIDNOTFIND
+    b.close()
+    mat.close()
 
 
 @pytest.mark.parametrize("seed", range(2))
