@@ -87,6 +87,7 @@ struct Status
    // some did not fit
    int32_t listed[2];
    int32_t listovf[2];
+   unsigned long long chgbase;       // the sum of slot_chg at the start of the round
    Counter wlcount[2][SAP_NBINS];    // worklist lengths (what did not fit is counted too)
    Counter touched;                  // touched-column count (likewise)
    unsigned long long rows_swept;
@@ -97,7 +98,6 @@ struct Status
    unsigned long long slot_nnz[SAP_STAT_SLOTS];
    unsigned long long slot_rows[SAP_STAT_SLOTS];
    Sum slot_chg[SAP_CHG_SLOTS];      // changed bounds: few, so that the marking can read them all
-   unsigned long long chgbase;       // their sum at the start of the round
    // sweep launch duration from the constant-rate wall clock: earliest workgroup start and
    // latest workgroup end per slot, folded at the end of the round
    unsigned long long tslot0[SAP_STAT_SLOTS];
@@ -2719,10 +2719,14 @@ __device__ __forceinline__ void noteMarked(Status* st, int32_t next, bool anymar
       st->anymark[next & 1] = 1;
 }
 
+// D: a dense set; a sparse one's rounds are all listed, from the touched columns
+template <bool D>
 __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
 {
    Status* st = V.st;
    const int t = (int)threadIdx.x;
+   const RoundView rv = roundView(V);
+   const unsigned long long before = st->chgbase;   // on the line of the round's fields
    // the tag of the thread's first column and the round's changed bounds (SAP_CHG_SLOTS lines that
    // other XCDs have just added to: 1 us) are asked for together with the round's fields, and the
    // count is waited for last: a scanned round's marking 10.6 -> 10.4 us (100,000 rows, first
@@ -2731,14 +2735,13 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
    // as the sweep's statistics took barriers, 5-7 us
    const size_t n = (size_t)V.nvec * (size_t)M.ncols;
    const size_t flat0 = blockIdx.x * (size_t)SAP_BLOCK + t;
+   const bool early = D && n <= (size_t)gridDim.x * SAP_BLOCK;   // the thread's only column
    int32_t tag0 = 0;
-   if( V.dense && flat0 < n )
+   if( early && flat0 < n )
       tag0 = V.chgtag[flat0];
    unsigned long long changed = 0;
-   if( V.dense && (t & (SAP_WAVE - 1)) < SAP_CHG_SLOTS )
+   if( D && (t & (SAP_WAVE - 1)) < SAP_CHG_SLOTS )
       changed = st->slot_chg[t & (SAP_WAVE - 1)].n;
-   const unsigned long long before = st->chgbase;
-   const RoundView rv = roundView(V);
    if( rv.done || (V.single && rv.cutoff) )
       return;
    __shared__ MarkShared S;
@@ -2748,10 +2751,10 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
    const int32_t next = round + 1;
    bool anymarked = false;
    bool list = true;
-   if( rv.columns )
+   if( !D || rv.columns )
    {
       const uint32_t n = rv.touched;
-      list = !V.dense || (uint64_t)n <= (uint64_t)V.listper * (uint64_t)V.nvec;
+      list = !D || (uint64_t)n <= (uint64_t)V.listper * (uint64_t)V.nvec;
       // the loop is workgroup-uniform: st->touched is not written in this launch
       for( uint32_t c0 = blockIdx.x * SAP_BLOCK; c0 < n; c0 += gridDim.x * SAP_BLOCK )
       {
@@ -2784,6 +2787,8 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
       // the first column's rows are looked up before the count is waited for
       int64_t beg0 = 0, end0 = 0;
       int32_t v0 = 0;
+      if( !early && flat0 < n )
+         tag0 = V.chgtag[flat0];
       if( flat0 < n && tag0 == round )
          changedRows(M, V, flat0, beg0, end0, v0);
 #pragma unroll
@@ -2842,14 +2847,15 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
          }
       }
    }
-   if( V.dense && blockIdx.x == 0 && t == 0 )
+   if( D && blockIdx.x == 0 && t == 0 )
       st->listed[next & 1] = list ? 1 : 0;
    noteMarked(st, next, anymarked);
 }
 
+template <bool D>
 __global__ __launch_bounds__(SAP_BLOCK, 8) void k_mark(Mat M, Vec V)
 {
-   markRound(M, V);
+   markRound<D>(M, V);
 }
 
 // ... of a dense set that never lists (listLimits): without the count, the lists and their LDS,
@@ -5155,7 +5161,10 @@ static void boundsRelease(sap_bounds* b)
 //     wavefront, 10-14 us, and a list saves 0-2 us of that and costs its marking 3.5 us (50,000
 //     rows, 2,660 tiles: two rounds listed 7.8 + 6.4 us of marking and 14.0 + 10.4 of sweeps,
 //     scanned 5.1 + 4.5 and 14.2 + 12.7; 80,000 rows, 4,260 tiles: equal; 100,000 rows, 5,325
-//     tiles: the sweeps 15 + 11 instead of 22 + 14 us).
+//     tiles: the sweeps 15 + 11 instead of 22 + 14 us).  Sets of several vectors serve calls from a
+//     fixpoint, all of whose rounds are small and the first of which is listed from the overlays:
+//     for them half as many tiles (50 vectors of 1,017 rows, 2,600 tiles, three rounds: 14.6 + 12.1 +
+//     11.0 us of sweeps listed, 16.7 + 15.4 + 14.3 scanned, and 4 us less of marking).
 // 200 strong-branching children of 20,011 rows take 310 us (555-597 us scanned), a node of
 // 148,409 rows among 31 a third of what it took.
 #define SAP_LIST_ROWS ((uint32_t)1 << 17)
@@ -5170,7 +5179,7 @@ static void listLimits(const sap_matrix* m, Vec& V)
       return;
    V.listcap = SAP_LIST_ROWS;
    V.touchcap = SAP_LIST_COLS;
-   if( (int64_t)V.nvec * m->ntiles <= SAP_LIST_TILES )
+   if( (int64_t)V.nvec * m->ntiles <= (V.nvec > 1 ? SAP_LIST_TILES / 2 : SAP_LIST_TILES) )
       return;
    const double deg = m->ncols > 0 ? (double)m->nnz / (double)m->ncols : 0.0;
    V.listper = (uint32_t)std::max(1.0, std::min(1e9, (double)m->nrows / 64.0 / std::max(deg, 1.0)));
@@ -5751,8 +5760,10 @@ static void enqueueRound(sap_bounds* b, const Mat& M, const Params& P, const Lay
    }
    if( b->V.dense && b->V.listper == 0 )
       k_mark_tags<<<colgrid, SAP_BLOCK, 0, s>>>(M, b->V);
+   else if( b->V.dense )
+      k_mark<true><<<colgrid, SAP_BLOCK, 0, s>>>(M, b->V);
    else
-      k_mark<<<colgrid, SAP_BLOCK, 0, s>>>(M, b->V);
+      k_mark<false><<<colgrid, SAP_BLOCK, 0, s>>>(M, b->V);
 }
 
 // ranged-row propagation keeps one check-group flag per (vector, nonzero); allocated on the
