@@ -2730,18 +2730,23 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
    // the tag of the thread's first column and the round's changed bounds (SAP_CHG_SLOTS lines that
    // other XCDs have just added to: 1 us) are asked for together with the round's fields, and the
    // count is waited for last: a scanned round's marking 10.6 -> 10.4 us (100,000 rows, first
-   // round), 12.2 us when the count came first.  The count is exact: a sample of the columns
-   // mistook changes that cluster by column (282 -> 490 us a call), and a count over as many slots
-   // as the sweep's statistics took barriers, 5-7 us
+   // round), 12.2 us when the count came first.  Calls on several vectors mostly list their rounds,
+   // which need neither.  The count is exact: a sample of the columns mistook changes that
+   // cluster by column (282 -> 490 us a call), and a count over as many slots as the sweep's
+   // statistics took barriers, 5-7 us
    const size_t n = (size_t)V.nvec * (size_t)M.ncols;
    const size_t flat0 = blockIdx.x * (size_t)SAP_BLOCK + t;
-   const bool early = D && n <= (size_t)gridDim.x * SAP_BLOCK;   // the thread's only column
+   const bool early = D && V.nvec == 1;
    int32_t tag0 = 0;
-   if( early && flat0 < n )
-      tag0 = V.chgtag[flat0];
    unsigned long long changed = 0;
-   if( D && (t & (SAP_WAVE - 1)) < SAP_CHG_SLOTS )
-      changed = st->slot_chg[t & (SAP_WAVE - 1)].n;
+   auto ask = [&]() {
+      if( flat0 < n )
+         tag0 = V.chgtag[flat0];
+      if( (t & (SAP_WAVE - 1)) < SAP_CHG_SLOTS )
+         changed = st->slot_chg[t & (SAP_WAVE - 1)].n;
+   };
+   if( early )
+      ask();
    if( rv.done || (V.single && rv.cutoff) )
       return;
    __shared__ MarkShared S;
@@ -2787,8 +2792,8 @@ __device__ __forceinline__ void markRound(const Mat& M, const Vec& V)
       // the first column's rows are looked up before the count is waited for
       int64_t beg0 = 0, end0 = 0;
       int32_t v0 = 0;
-      if( !early && flat0 < n )
-         tag0 = V.chgtag[flat0];
+      if( !early )
+         ask();
       if( flat0 < n && tag0 == round )
          changedRows(M, V, flat0, beg0, end0, v0);
 #pragma unroll
