@@ -349,8 +349,8 @@ int sap_slots_collect(sap_bounds* bnd, int32_t n, const int32_t* slots, int32_t*
  * maxneghuge}, maxactdelta as in consdataRecomputeMaxActivityDelta (cons_linear.c:1542).
  * Any output pointer may be NULL. */
 /* sap_propagate on bounds already in device memory, allocating nothing.  No counterpart in
- * SCIP: it is for callers that cannot allocate device memory (code under HIP graph capture,
- * tight serving loops, harnesses that forbid hipMalloc).  dlb and dub are device pointers to
+ * SCIP: it is for callers that cannot allocate device memory (tight serving loops, harnesses
+ * that forbid hipMalloc); it waits on its stream, so it cannot be part of a captured graph.  dlb and dub are device pointers to
  * ncols doubles, the node's bounds, overwritten with the fixpoint unless the result is a
  * cutoff.  The work arrays live in one static device array per GPU (about 66 MiB, held until
  * the process ends), so the matrix may have at most 2^20 columns and 2^20 rows and one

@@ -17,7 +17,9 @@
 //                   (scip_var.c:6965-7174) to its tightest regular and forced candidates and
 //                   writes the new bounds.
 //   k_mark        : the rows of changed columns (CSC) are marked for the next round (dense
-//                   mode) or appended to its per-bin worklists (sparse mode).
+//                   mode), appended to its per-bin worklists (sparse mode), or both (dense
+//                   sets of many tiles after a round of few changes); k_mark_tags in dense
+//                   sets that never keep lists.
 // Rounds run in groups of 1 (enqueued directly), then 2, 4 and 8 (captured graphs); the host
 // applies the same stop test as k_round_begin to the status it reads back after each group.
 //
@@ -3860,9 +3862,9 @@ __global__ void k_noalloc_begin(Vec V, const double* lb, const double* ub, int64
 }
 
 // the status of a call on vector 0, written to mapped host memory after every round group (hst
-// NULL: not asked for), and its outcome once the call has ended (its done flag, or the stop test the host applies after the group): the
-// bounds (lb NULL: not asked for), and the first histmax entries of the reason history as 32-bit
-// words (hist NULL: none)
+// NULL: not asked for), and its outcome once the call has ended (its done flag, or the stop test
+// that the host applies after the group): the bounds, and the first histmax entries of the
+// reason history as 32-bit words (hist NULL: none)
 __global__ void k_land(Vec V, int64_t ncols, int32_t maxrounds, uint32_t* hst, double* lb, double* ub, uint32_t* hist,
    uint32_t histmax)
 {
@@ -3949,7 +3951,8 @@ __global__ __launch_bounds__(SAP_BLOCK) void k_row_activities(Mat M, Params P, c
 // ---- scratch of the no-allocation entry point (sap_propagate_device_noalloc) ----
 // One dense single-vector bound set (bounds, candidate keys, round tags, row marks, redundancy
 // flags, per-unit counters and the status block) for matrices of up to SAP_NOALLOC_MAXCOLS
-// columns and SAP_NOALLOC_MAXROWS rows: 56 B per column, 5 B per row, 256-byte aligned pieces.
+// columns and SAP_NOALLOC_MAXROWS rows: 56 B per column, 5 B per row, 19 lists of
+// SAP_NOALLOC_LIST entries (4.75 MiB) and the status, in 256-byte aligned pieces.
 #define SAP_NOALLOC_MAXCOLS ((int64_t)1 << 20)
 #define SAP_NOALLOC_MAXROWS ((int64_t)1 << 20)
 #define SAP_NOALLOC_LIST ((uint32_t)1 << 15)   // entries of each worklist
@@ -5400,9 +5403,8 @@ struct Helpers
 // SAP_RING_COLS columns go through pinned staging and one kernel that reads it, with no wait
 // (two pageable copies waited 10-20 us each): the caller's later wait covers it.  With the
 // result landing by the call's own wait as well, sap_propagate on 2,000 x 5,000 went from 135 to
-// 87 us.  Longer arrays
-// are copied by the runtime, which reads pageable memory at the link's rate (25 us a MiB),
-// while helper threads look for NaNs.  room: staging the caller needs behind the arrays.
+// 87 us.  Longer arrays are copied by the runtime, which reads pageable memory at the link's rate
+// (25 us a MiB), while helper threads look for NaNs.  room: staging the caller needs behind the arrays.
 // defer: the next beginCall takes the staged arrays over, without a launch of its own.
 static int uploadBounds(sap_bounds* b, int32_t v, const double* lb, const double* ub, size_t room = 0, bool defer = false)
 {
@@ -5993,8 +5995,8 @@ static int runRounds(sap_bounds* b, const Params& P, sap_stats* stats, int32_t m
       if( land != NULL )
          RCCHK(enqueueLand(b, P, land, c->hstatusd));
       else
-         k_copy_words<<<gridFor(sizeof(Status) / 4), SAP_BLOCK, 0, s>>>((uint32_t*)c->hstatusd, (const uint32_t*)b->dstatus,
-         sizeof(Status) / 4);
+         k_copy_words<<<gridFor(sizeof(Status) / 4), SAP_BLOCK, 0, s>>>((uint32_t*)c->hstatusd,
+            (const uint32_t*)b->dstatus, sizeof(Status) / 4);
       if( metan > 0 )
          k_pack_meta<<<gridFor((size_t)metan), SAP_BLOCK, 0, s>>>(b->V, metan, (int32_t*)b->hdnd);
       HIPCHK(hipGetLastError());
