@@ -5643,9 +5643,11 @@ static Layout makeLayout(const sap_bounds* b)
    // with many per wavefront (1M rows, 12.7) the places cost the tiles more than the tail.
    // The tiles' workgroups start in ascending order, those with one tile more than the others first:
    // in descending order that tile was the tail (first sweep of 80,000 rows 45 instead of 37 us, of
-   // 300,000 rows 95 instead of 83 us).  Where nearly all have it, descending order measured
-   // better, for a reason not found (130,000 rows, 1.9 tiles: 199 us ascending, 189 us descending;
-   // 200,000 rows, 2.9: 261 and 252 us), so that remains above 4/5 of the wavefronts.
+   // 300,000 rows 95 instead of 83 us).  Once more than about three workgroups of a CU's four have
+   // it, ascending order puts four of them on some CUs, and descending order measures better.
+   // Sweeps of a call, ascending / descending: 116,000 rows (1.68 tiles per wavefront) 179 / 183
+   // us, 120,000 (1.74) 190 / 184, 190,000 (2.75) 242 / 244, 195,000 (2.82) 262 / 251, 262,000 (3.79)
+   // 294 / 303, 266,000 (3.85) 325 / 313, 330,000 (4.77) 354 / 367, 335,000 (4.85) 376 / 364 us.
    const size_t res = (size_t)std::max(m->ctx->resident, 0);
    L.longfirst = L.tilesdown = 0;
    if( b->V.dense && res > 0 && blocks[0] > 0 )
@@ -5663,7 +5665,7 @@ static Layout makeLayout(const sap_bounds* b)
          room = std::max(res / 2, others < res ? res - others : 0);
          L.longfirst = 1;
          const size_t tiles = units[0] / (size_t)kUnits[0], waves = room * (SAP_BLOCK / SAP_WAVE);
-         L.tilesdown = 5 * (tiles % waves) > 4 * waves ? 1 : 0;
+         L.tilesdown = 10 * (tiles % waves) > (tiles < 2 * waves ? 7 : 8) * waves ? 1 : 0;
       }
       blocks[0] = std::min(blocks[0], room);
    }
