@@ -120,7 +120,9 @@ int64_t footprint(const Problem* p, int32_t slots)
    const int64_t nnz = p->rowptr.empty() ? 0 : p->rowptr.back();
    const int64_t mat = nnz * (8 + 4 + 4 + 1) + nnz / 4 + p->nrows * (8 + 16 + 1 + 1 + 1 + 4 + 4 + 8) + p->ncols * (1 + 8 + 4)
       + 4096;
-   const int64_t vec1 = p->ncols * (16 + 16 + 16 + 4 + 4 + 32) + p->nrows * (4 + 1 + 16);
+   // the root is a dense set: its touched list holds at most 65,536 columns (8 B each)
+   const int64_t vec1 = p->ncols * (16 + 16 + 16 + 4 + 4 + 32) + p->nrows * (4 + 1 + 16)
+      + 8 * std::min<int64_t>(p->ncols, 65536);
    const int64_t pool = (int64_t)slots * (p->ncols * (16 + 16 + 16 + 4 + 4 + 8 + 4 + 4 + 1) + p->nrows * (4 + 1 + 16))
       + p->ncols * 32 + 65536;
    return mat + vec1 + pool;
